@@ -85,6 +85,8 @@ def draw(rng):
     if kind == "prefill":
         rows = _log_int(rng, 16, 4096)
         pos0 = rng.choice([0, rng.randrange(1, 512), _log_int(rng, 64, 16384)])
+        most = 32 * 8192 * 8192 // 2 // heads  # query-key pairs per head of the largest listed case
+        pos0 = max(0, min(pos0, most // rows - rows))
         return dict(kind=kind, heads=heads, kv_heads=kv_heads, rows=rows, pos0=pos0, block=rng.choice([0, 0, 0, 64]))
     n_embd, n_out = rng.choice([(1024, 4096), (2048, 4096), (2560, 6144), (4096, 6144), (5120, 7168)])
     return dict(kind=kind, n_embd=n_embd, n_out=n_out, rows=rng.choice([1, 1, 2, 3, 4]), layers=rng.choice([1, 4, 12]),
