@@ -1,19 +1,25 @@
-// prefill.hip — causal GQA prefill attention on gfx950 fp32 matrix cores.
+// prefill.hip — causal GQA prefill attention on gfx950 bf16 matrix cores, fp32-exact operands.
 //
-// Contraction on v_mfma_f32_32x32x2_f32 (fp32 inputs, fp32 accumulate; 4096 FLOP per
-// instruction), online softmax in fp32 VALU between the two products.
+// Both products run on v_mfma_f32_32x32x16_bf16 (fp32 accumulate; 16x the rate of the fp32
+// 32x32x2 instruction) with every fp32 operand split into three bf16 planes that together hold
+// all of its bits, x = h + m + l.  Six of the nine plane products are taken; the three left out
+// are each at most 2^-27 of |a||b|, an eighth of an fp32 rounding.  An instruction sums 16
+// products before it rounds, so a 128-deep score takes 48 roundings, most of them of small
+// terms, against 64 on the fp32 instruction.  Measured error of the output against 64 bits
+// (2-norm): 3.3e-7 against 4.0e-7 with fp32 MFMA (2048-token prompt, H32/HKV8), 4.4e-7 against
+// 5.2e-7 (8192 tokens), 6.1e-7 against 7.1e-7 (512 tokens at 7680, H16/HKV8); lower in every
+// shape tried.  Online softmax in fp32 VALU between the two products.
 //
 // Each wave owns 32 queries of one head.  It computes the transposed score tile
-//     S^T[key][query] = K . Q^T          (A = K rows from LDS, B = Q^T held in registers)
+//     S^T[key][query] = K . Q^T          (A = K planes from LDS, B = Q^T planes in registers)
 // so that in the 32x32 accumulator layout every lane owns ONE query column and 16 key
 // rows: the row max / row sum of the softmax need only the lane's own 16 values plus one
-// exchange with lane^32.  The same registers, unchanged, are the B operand of
-//     O^T[d][query] = V^T . P^T          (A = V from LDS)
+// exchange with lane^32.  The same registers, split into planes, are the B operand of
+//     O^T[d][query] = V^T . P^T          (A = transposed V planes from LDS)
 // because the accumulator row order (8*(r/4) + 4*(lane/32) + r%4) is used as the
-// contraction order of the second product.  In the first product, step 4*k4 + j of lane
-// half hh contracts d = 8*k4 + 4*hh + j.
-// Output block db (0..3) of O^T holds d = 4*i + db for accumulator row i, so the A operand
-// of all four blocks for one key is a single 16-byte LDS read V[key][4*lane .. 4*lane+3].
+// contraction order of the second product: step s of lane half hh takes registers 8s .. 8s+7,
+// keys 16s + 4hh + {0..3, 8..11}, and the V planes are stored with those eight keys side by
+// side.  Output block db (0..3) of O^T holds d = 32*db + i for accumulator row i.
 //
 // Workgroup = KS key groups x 4 query slots of one KV head.  A slot is one (query block,
 // head) pair; slots are numbered s = qb*G + g over the G heads that share the KV head, and
@@ -22,33 +28,37 @@
 // four neighbouring blocks of the head, for odd G at most two neighbouring blocks: every
 // wave of the unit shares every K/V tile, and the unit's key range ends at its last
 // block's diagonal (a wave of an earlier block masks the few tiles past its own).  Slots
-// past the last block are idle waves (zero queries, no output).  Key group g takes the
+// past the last block repeat a valid row and write nothing.  Key group g takes the
 // tiles kt = KS*i + g of the unit's causal range and keeps its own (m, l, O); the groups
-// merge through LDS at the end of the unit.  With KS = 2 every SIMD runs two waves whose
-// matrix streams interleave: one streams while the other waits on LDS or the per-tile
-// barrier (their VALU work still adds to the matrix time: on this part a wave's fp32 MFMA
-// stream holds the SIMD's issue).  Inside a wave's stream the next score chain alternates
-// with this tile's P.V chains, and the next tiles' DMA instructions are issued between them
-// (VMEM work outside the stream idles the pipe).  When one unit pair per KV head would not
+// merge through LDS at the end of the unit.  When one unit pair per KV head would not
 // fill the CUs (short chunks at long positions, GQA groups under 4 heads;
 // ei_attn_prefill_split) the pair's key tiles are split over ksplit workgroups of equal cost
 // (a share that crosses from one unit to the other pays a second pass), whose unnormalised
 // shares k_prefill_combine merges.
 //
-// K/V tiles (32 keys) reach LDS by LDS DMA (global_load_lds_dwordx4) straight from the
-// cache, two tiles ahead for K and one for V, per key group:
-//   K tile row-major, rows padded to 132 floats: the 32 lanes reading one 16-byte d-chunk
-//     of 32 different keys hit 32 distinct bank quads; each row is one 32-lane DMA
-//     instruction (a contiguous 512-byte global read: LDS DMA of 16-byte pieces gathered
-//     from many rows runs ~3.5x slower per CU than contiguous DMA);
-//   V tile row-major    [32 keys][128 floats], two rows per 64-lane DMA instruction.
-// Rows past the causal end are clamped to the last visible row (valid memory, masked out).
+// The key loop.  A tile (32 keys) is loaded by the four waves of its group, a quarter each, 16
+// floats of K or V per lane, split in registers and stored as planes (K [key][d], V transposed
+// [d][key]; rows padded to an odd number of 16-byte pieces).  Per half iteration a group either
+// multiplies K by Q, while V of the same tile goes to its planes and K of the next is fetched, or
+// runs the softmax and multiplies V by P, while the next K goes to its planes and the next V is
+// fetched: one set of planes per group and one set of 16 landing registers suffice, and a fetch
+// has half a phase and more to land.  The two groups run half an iteration apart, so of a SIMD's
+// two waves one has matrix work while the other is in its softmax (1-3% faster than in step; the
+// raised wave priority of the softmax half, whose chain is the longer one, another 3%).  Each
+// matrix step refills its three LDS operands right after their last use (mfma_split).
+//
+// What bounds it: the matrix power of the part.  At 8192 tokens (H32/HKV8) the kernel runs 217
+// TFLOP/s of attention = 1.30 PFLOP/s of bf16 MFMA at 1.65 GHz (the clock gives way under bf16
+// load: a bare register-to-register MFMA loop on random bits reaches 1.53-1.63 PFLOP/s at
+// 1.6-1.66 GHz), against 139 TFLOP/s on fp32 MFMA; 2048 tokens 285 -> 188 us a step, 512 tokens
+// at 7680 (H16/HKV8) 268 -> 160 us.  With parts taken out (timing only): without the K/V split
+// and its loads 2.14 ms of 2.53, without the loads alone 2.38, without operand reads as well as
+// the split 2.04, without the exponentials too 1.98.
+//
 // q and the output pass through LDS too, so that global memory sees whole 512-byte rows:
 // at the start of each unit the workgroup DMAs its 128 query rows (once, for both key
 // groups) into a padded staging area and each wave reads its Q^T operand from there; at the
 // end the finished rows are written there in row order and stored two rows per instruction.
-// (Gathering q straight into registers, 32 bytes per row per instruction, twice, and storing
-// 8-byte pieces of 32 rows per instruction held each pass up for several microseconds.)
 //
 // Softmax runs in the exp2 domain (scores x scale x log2 e, one FMA per score).  The
 // running maximum is raised only when a tile's maximum exceeds it by more than kLazy
@@ -71,10 +81,11 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int kQB = 32;                          // queries per wave (and per block)
 constexpr int kKT = 32;                          // keys per tile
-constexpr int kKS_F = kHeadDim + 4;             // padded K row (floats)
-constexpr int kKTileF = kKT * kKS_F;             // floats in one K tile
-constexpr int kVTileF = kKT * kHeadDim;          // floats in one V tile (16 KB)
-constexpr int kGroupF = 2 * kKTileF + 2 * kVTileF;  // per key group: 2 K + 2 V tile buffers
+constexpr int kKS_F = kHeadDim + 4;             // padded fp32 row of the staging area (floats)
+// plane rows are padded to an odd number of 16-byte pieces: the lanes of an operand read, one row
+// each, spread over all LDS banks
+constexpr int kKRowB = 2 * kHeadDim + 16, kKPlane = kKT * kKRowB;  // K plane: [32 keys][128 d] bf16
+constexpr int kVRowB = 2 * kKT + 16, kVPlane = kHeadDim * kVRowB;   // V plane, transposed: [128 d][32 keys] bf16
 constexpr int kKS = 2;                           // key groups per workgroup
 constexpr float kLazy = 8.f;                     // lazy-rescale threshold (log2 units)
 constexpr int kXchF = 34;                        // floats per lane exchanged by the merge
@@ -117,18 +128,14 @@ __device__ __forceinline__ void prefill_share(int pair, int u_second, int split,
     r1 = max(hi - max(lo, n0), 0);
 }
 
-// LDS (plain kernel): the four K tile buffers (two per key group) from 0; the merge exchange
-// area from 0 as well (used only after the unit's last tile); the four V tile buffers and,
-// overlapping them, the q staging area (the unit's 4 x 32 query rows, padded like K rows)
-// after the exchange area.  A unit's q rows and its first two K tiles land at the same time;
-// its first V tile is fetched once q has moved to registers.  (The kernel that norms q keeps
-// each key group's K0 K1 V0 V1 side by side from 0, and fetches the tiles after q.)
+// LDS: both key groups' K planes from 0, and the merge exchange area from 0 as well (used only
+// after the unit's last tile); after it both groups' V planes and, overlapping them, the staging
+// area (the unit's 4 x 32 query rows, later its output rows, in fp32, padded).  K planes are stored
+// while the query rows are staged, V planes once every wave has its query operand.
 constexpr int kQStageF = 2 * kSlots * kXchF * 64;
-constexpr int kVBaseF = kQStageF;
 constexpr int kLdsF = kQStageF + kSlots * kQB * kKS_F;
-static_assert(kKS * 2 * kKTileF <= kVBaseF, "K buffers below the V buffers and the q staging area");
-static_assert(kVBaseF + kKS * 2 * kVTileF <= kLdsF, "V buffers within the staging span");
-static_assert(kKS * kGroupF <= kLdsF, "grouped layout within the LDS budget");
+static_assert(kKS * 3 * kKPlane <= kQStageF * 4, "K planes below the staging area");
+static_assert(kQStageF * 4 + kKS * 3 * kVPlane <= kLdsF * 4, "V planes within the LDS span");
 
 // QK-norm + RoPE of one q row in LDS (rope_dim = 128), eight lanes per row: lane k of the row
 // holds elements 8k..8k+7 and their rotate-half partners 64+8k..64+8k+7.  Same arithmetic as the
@@ -174,18 +181,75 @@ __device__ __forceinline__ void norm_rope_q8(float* row, const float (&g)[16], c
     }
 }
 
-#ifdef EI_EXP_STAMPS
-__device__ unsigned long long g_pstamps[4096 * 16];
-#define PSTAMP(i) do { if (threadIdx.x == 0) g_pstamps[blockIdx.x * 16 + (i)] = __builtin_amdgcn_s_memtime(); } while (0)
-#define PSTAMPV(i, v) do { if (threadIdx.x == 0) g_pstamps[blockIdx.x * 16 + (i)] = (unsigned long long)(v); } while (0)
-#else
-#define PSTAMP(i) do { } while (0)
-#define PSTAMPV(i, v) do { } while (0)
-#endif
+// ------------------------------------------------------------------ three-plane split
+// x = h + m + l with h, m, l in bf16: h = bf16(x), m = bf16(x - h), l = x - h - m, each rounded to
+// nearest.  Both differences are exact (the residual of a 24-bit value rounded to 8 bits has at
+// most 16 significant bits, the second at most 8), so the three planes hold every bit of x.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+constexpr int kBufferDword3 = 0x00020000;  // raw 32-bit data, gfx9-family buffer resource word 3
+
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+#pragma clang fp contract(off)
+    h = pk_bf16(a, b);
+    const float ra = a - __uint_as_float(h << 16), rb = b - __uint_as_float(h & 0xFFFF0000u);
+    m = pk_bf16(ra, rb);
+    l = pk_bf16(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xFFFF0000u));
+}
+struct Planes {  // eight values: one MFMA operand per plane
+    u32x4 h, m, l;
+};
+__device__ __forceinline__ floatx16 mfma_bf16(u32x4 a, u32x4 b, floatx16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
+                                                   0, 0);
+}
+// c += a . b to 2^-26 of |a||b|: the six products of planes above that (m.l, l.m and l.l are
+// each at most 2^-27).  a's planes are used up one after another, and next(x) refills plane x
+// (2 l, 1 m, 0 h) with the next step's right after its last use: at least three matrix
+// instructions cover each LDS read, in the registers of one step.
+template <typename Next>
+__device__ __forceinline__ void mfma_split(Planes& a, const Planes& b, floatx16& c, Next next) {
+    constexpr int kAlu = 0x6;  // VALU and SALU work may move across, LDS reads and MFMAs stay in order
+    c = mfma_bf16(a.l, b.h, c);
+    __builtin_amdgcn_sched_barrier(kAlu);
+    a.l = next(2);
+    __builtin_amdgcn_sched_barrier(kAlu);
+    c = mfma_bf16(a.m, b.m, c);
+    c = mfma_bf16(a.m, b.h, c);
+    __builtin_amdgcn_sched_barrier(kAlu);
+    a.m = next(1);
+    __builtin_amdgcn_sched_barrier(kAlu);
+    c = mfma_bf16(a.h, b.l, c);
+    c = mfma_bf16(a.h, b.m, c);
+    c = mfma_bf16(a.h, b.h, c);
+    __builtin_amdgcn_sched_barrier(kAlu);
+    a.h = next(0);
+    __builtin_amdgcn_sched_barrier(kAlu);
+}
+
+// A value the optimiser may not carry across loop iterations: what is derived from it is computed
+// where it is used (the vector registers of the key loop are full, hoisted addresses would spill).
+__device__ __forceinline__ int unhoisted(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
+// Workgroup barrier ordering LDS only: global loads stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
 // kPaged: key t of the sequence sits in pool row btab[t >> bshift] << bshift | (t & mask), the
 // block size 2^bshift >= 32, so a 32-key tile lies in one block and its rows are consecutive.
-template <bool kNormQ, bool kPaged, bool kEarlyK = false>
+template <bool kNormQ, bool kPaged>
 __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __restrict__ q, long q_stride,
                                                            float* __restrict__ out, const float* __restrict__ kc,
                                                            const float* __restrict__ vc,
@@ -198,10 +262,8 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
                                                            int max_blocks) {
     constexpr int D = kHeadDim;
     constexpr int GW = kSlots;
-    constexpr int DMA_PER_WAVE = 16 / GW;  // V DMA instructions per wave per tile (K: twice as many, 32 lanes each)
     extern __shared__ __align__(16) float smem[];
 
-    PSTAMP(0);
     const int L = blockIdx.x;
     const int kvh = L % HKV;
     const int rest = L / HKV;
@@ -217,7 +279,6 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
     const size_t KD = (size_t)HKV * D;
     const float* kbase = kc + (size_t)kvh * D;
     const float* vbase = vc + (size_t)kvh * D;
-    const uint64_t kb_bytes = (uint64_t)(uintptr_t)kbase, vb_bytes = (uint64_t)(uintptr_t)vbase;
     const uint32_t row_bytes = (uint32_t)(KD * sizeof(float));          // one cache row (all KV heads)
     // cache row of key t (wave-uniform t: one scalar load of the block table when paged)
     auto crow = [&](int t) -> uint32_t {
@@ -226,24 +287,24 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
             return ((uint32_t)btab[min(t >> bshift, max_blocks - 1)] << bshift) | ((uint32_t)t & ((1u << bshift) - 1u));
         else return (uint32_t)t;
     };
-    const uint32_t voff_k = 16u * col;                                  // K: lanes 0..31, one row
-    const uint32_t voff_v = (uint32_t)hh * row_bytes + 16u * col;        // V: two rows per instruction
     const int nb = (B + kQB - 1) / kQB;
     const int nslot = G * nb;                    // (block, head) slots of this KV head
     const int nu = (nslot + kSlots - 1) / kSlots;  // units
-    // this key group's K0 K1 and V0 V1: K buffers below the staging area for the plain kernel,
-    // which fetches q and the first K tiles together; with the in-kernel q norm (q first,
-    // then the tiles) a group's four buffers side by side measured 0.7% faster
-    constexpr bool kGrouped = kNormQ && !kEarlyK;
-    float* gsm = kGrouped ? smem + grp * kGroupF : smem + grp * 2 * kKTileF;
-    float* gsv = kGrouped ? gsm + 2 * kKTileF : smem + kVBaseF + grp * 2 * kVTileF;
+    char* const lds = reinterpret_cast<char*>(smem);
+    char* const kpl = lds + grp * 3 * kKPlane;                 // this key group's K planes
+    char* const vpl = lds + kQStageF * 4 + grp * 3 * kVPlane;  // and its V planes
     const float sl2 = scale * 1.44269504088896340736f;
+    const uint32_t voff_k = (uint32_t)(8 * hw + (lane >> 3)) * row_bytes + 32u * (lane & 7);
+    const uint32_t voff_v =
+        (uint32_t)(16 * (lane >> 5) + 4 * ((lane >> 4) & 1)) * row_bytes + 4u * (32 * hw + 2 * (lane & 15));
 
     // q of unit u reaches LDS by LDS DMA, once per workgroup: row r = 32*slot + j holds query
     // qb*32 + j of the slot's head (one contiguous 512-byte DMA per row; rows past B and idle
     // slots are clamped to valid rows, never written out).  Both key groups then read their
-    // Q^T operand from it: qreg[4*k4 + j] = q[qb*32 + col][h][8*k4 + 4*hh + j].
+    // Q^T operand from it and split it into planes: step t holds d = 16t + 8hh .. + 7 of query
+    // qb*32 + col.
     float* qst = smem + kQStageF;
+    const uint32_t voff_q = 16u * col;
     // wave wu stages rows 16*wu .. 16*wu+15 of unit u: half of slot wu/2, query rows r0 + min(j, jm)
     auto stage_rows = [&](int u, int& r0, int& jm, int& hq) {
         const int sl = kSlots * u + (wu >> 1);
@@ -263,12 +324,12 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
         if (hh == 0) {
 #pragma unroll
             for (int j = 0; j < kQB / 2; ++j) {
-                dma16_s(sb, voff_k, lb + j * (kKS_F * 4));
+                dma16_s(sb, voff_q, lb + j * (kKS_F * 4));
                 if (j < jm) sb += rs;
             }
         }
     };
-    float qreg[64];
+    Planes qp[8];
     // raw q rows (kNormQ): QK-norm + RoPE in place, each wave on the 16 rows it staged, 8 lanes
     // per row, two rounds of 8 rows; gamma and both rounds' RoPE rows are loaded (load_norm)
     // while the q rows are still in flight, and used once they have landed (read_q)
@@ -304,15 +365,18 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
             for (int h = 0; h < 2; ++h)
                 norm_rope_q8(qst + ((kQB / 2) * wu + 8 * h + j) * kKS_F, qg, qt[h], eps, k);
         }
-        __syncthreads();
-        const float* qs = qst + (hw * kQB + col) * kKS_F + 4 * hh;
+        lds_barrier();
+        const float* qs = qst + (hw * kQB + col) * kKS_F + 8 * hh;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const float4 v = *reinterpret_cast<const float4*>(qs + 8 * i);
-            qreg[4 * i] = v.x;
-            qreg[4 * i + 1] = v.y;
-            qreg[4 * i + 2] = v.z;
-            qreg[4 * i + 3] = v.w;
+        for (int t = 0; t < 8; ++t) {
+            const float4 x = *reinterpret_cast<const float4*>(qs + 16 * t);
+            const float4 y = *reinterpret_cast<const float4*>(qs + 16 * t + 4);
+            uint32_t h[4], m[4], l[4];
+            split_pair(x.x, x.y, h[0], m[0], l[0]);
+            split_pair(x.z, x.w, h[1], m[1], l[1]);
+            split_pair(y.x, y.y, h[2], m[2], l[2]);
+            split_pair(y.z, y.w, h[3], m[3], l[3]);
+            qp[t] = {u32x4{h[0], h[1], h[2], h[3]}, u32x4{m[0], m[1], m[2], m[3]}, u32x4{l[0], l[1], l[2], l[3]}};
         }
     };
     const int u_second = nu - 1 - pair;  // the pass-1 unit (none when it equals pair)
@@ -325,8 +389,6 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
     lo1 = __builtin_amdgcn_readfirstlane(lo1);
     r1 = __builtin_amdgcn_readfirstlane(r1);
     const int npass = (r0 > 0) + (r1 > 0);
-    PSTAMPV(12, r0);
-    PSTAMPV(13, r1);
 
     for (int pass = 0; pass < npass; ++pass) {
         const bool first_unit = pass == 0 && r0 > 0;  // this pass runs unit `pair`
@@ -338,13 +400,6 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
         const int b = qb * kQB + col;  // this lane's query row
         const int qpos = pos0 + b;
 
-        floatx16 o[4];
-#pragma unroll
-        for (int db = 0; db < 4; ++db)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) o[db][i] = 0.f;
-        float m = -INFINITY, lsum = 0.f;
-
         const int T = pos0 + min(B, qb_last * kQB + kQB);  // keys seen by the unit's last query
         const int ntile = (T + kKT - 1) / kKT;
         const int nfull = live ? (pos0 + qb * kQB + 1) / kKT : ntile;  // tiles below this wave's diagonal
@@ -353,82 +408,92 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
         const int n_it = (nrange + kKS - 1) / kKS;
         const int n_mine = (nrange - grp + kKS - 1) / kKS;  // tiles of this key group
 
-        // DMA of this group's i-th tile (kt = KS*i + grp) into a K or V buffer
-        // DMA of this group's i-th tile (kt = KS*i + grp).  A tile wholly below T uses the
-        // scalar-base form with per-lane byte offsets fixed for the pass; the tile that
-        // reaches past T clamps each row to the last visible one (valid memory, masked out).
-        auto dma_k = [&](int i, int buf) {
-            const int t0 = (kt_lo + kKS * i + grp) * kKT;
-            const uint32_t lb = __builtin_amdgcn_readfirstlane(lds_addr(gsm + buf * kKTileF));
-            const int r0 = hw * 2 * DMA_PER_WAVE;  // this wave's first row of the tile
-            if (hh == 0) {
-                const uint32_t row0 = crow(t0);  // the tile's rows are consecutive from here
-                if (t0 + kKT <= T) {
-                    const uint64_t sb = kb_bytes + (uint64_t)(row0 + r0) * row_bytes;
+        // K and V of this group's i-th tile (kt = KS*i + grp): wave hw takes a quarter of each,
+        // 16 floats per lane, into rg, and stores them as planes.  Rows past T repeat the last
+        // visible one (valid memory, masked out).
+        //   K: row 8*hw + lane/8, d = 8c .. 8c+7 and 64 + 8c .. (c = lane%8): two 16-byte pieces
+        //     of a row per plane
+        //   V: d = 32*hw + 2*(lane%16) and the next, the eight keys of chunk lane/16 (step s =
+        //     chunk/2, half hh = chunk%2 of the P.V operand: keys 16s + 4hh + {0..3, 8..11}): one
+        //     16-byte piece of two transposed rows per plane
+        float rg[16];
+        // the tile's visible rows as a buffer: reads past the last one give zeros (masked out)
+        auto tile_rsrc = [&](const float* cache, int t0) {
+            return __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<float*>(cache) + (size_t)crow(t0) * KD, 0,
+                (int)((uint32_t)(min(kKT, T - t0) - 1) * row_bytes + D * 4), kBufferDword3);
+        };
+        auto load_k = [&](int i) {
+            const __amdgpu_buffer_rsrc_t rs = tile_rsrc(kbase, (kt_lo + kKS * i + grp) * kKT);
 #pragma unroll
-                    for (int j = 0; j < 2 * DMA_PER_WAVE; ++j)  // one padded row per instruction
-                        dma16_s(sb + (uint64_t)j * row_bytes, voff_k, lb + (r0 + j) * (kKS_F * 4));
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 2 * DMA_PER_WAVE; ++j) {
-                        const int key = min(t0 + r0 + j, T - 1);
-                        dma16(kbase + (size_t)(row0 + (key - t0)) * KD + 4 * col, lb + (r0 + j) * (kKS_F * 4));
-                    }
-                }
+            for (int j = 0; j < 4; ++j) {
+                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, voff_k + 256 * (j >> 1) + 16 * (j & 1), 0, 0);
+                rg[4 * j] = __uint_as_float(v.x), rg[4 * j + 1] = __uint_as_float(v.y);
+                rg[4 * j + 2] = __uint_as_float(v.z), rg[4 * j + 3] = __uint_as_float(v.w);
             }
         };
-        auto dma_v = [&](int i, int buf) {
-            const int t0 = (kt_lo + kKS * i + grp) * kKT;
-            const uint32_t lb = __builtin_amdgcn_readfirstlane(lds_addr(gsv + buf * kVTileF));
-            const int i0 = hw * DMA_PER_WAVE;  // 1 KB instruction = keys 2*ins, 2*ins+1
-            const uint32_t row0 = crow(t0);
-            if (t0 + kKT <= T) {
-                const uint64_t sb = vb_bytes + (uint64_t)(row0 + 2 * i0) * row_bytes;
+        auto load_v = [&](int i) {
+            const __amdgpu_buffer_rsrc_t rs = tile_rsrc(vbase, (kt_lo + kKS * i + grp) * kKT);
+            const uint32_t off = unhoisted(voff_v);
 #pragma unroll
-                for (int j = 0; j < DMA_PER_WAVE; ++j)
-                    dma16_s(sb + (uint64_t)(2 * j) * row_bytes, voff_v, lb + (i0 + j) * 1024);
-            } else {
-#pragma unroll
-                for (int j = 0; j < DMA_PER_WAVE; ++j) {
-                    const int key = min(t0 + 2 * (i0 + j) + hh, T - 1);
-                    dma16(vbase + (size_t)(row0 + (key - t0)) * KD + 4 * col, lb + (i0 + j) * 1024);
-                }
+            for (int j = 0; j < 8; ++j) {
+                const u32x2 v =
+                    __builtin_amdgcn_raw_buffer_load_b64(rs, off + (8 * (j >> 2) + (j & 3)) * row_bytes, 0, 0);
+                rg[2 * j] = __uint_as_float(v.x), rg[2 * j + 1] = __uint_as_float(v.y);
             }
+        };
+        // half x of the conversion of rg: eight values, one 16-byte piece of each plane
+        auto conv_k = [&](int x) {
+            uint32_t ch[4], cm[4], cl[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) split_pair(rg[8 * x + 2 * j], rg[8 * x + 2 * j + 1], ch[j], cm[j], cl[j]);
+            char* p = kpl + (8 * hw + (lane >> 3)) * kKRowB + 16 * (lane & 7) + 128 * x;
+            *reinterpret_cast<u32x4*>(p) = u32x4{ch[0], ch[1], ch[2], ch[3]};
+            *reinterpret_cast<u32x4*>(p + kKPlane) = u32x4{cm[0], cm[1], cm[2], cm[3]};
+            *reinterpret_cast<u32x4*>(p + 2 * kKPlane) = u32x4{cl[0], cl[1], cl[2], cl[3]};
+        };
+        auto conv_v = [&](int x) {  // d + x
+            uint32_t ch[4], cm[4], cl[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) split_pair(rg[4 * j + x], rg[4 * j + 2 + x], ch[j], cm[j], cl[j]);
+            char* p = vpl + (32 * hw + 2 * (lane & 15) + x) * kVRowB + 16 * (lane >> 4);
+            *reinterpret_cast<u32x4*>(p) = u32x4{ch[0], ch[1], ch[2], ch[3]};
+            *reinterpret_cast<u32x4*>(p + kVPlane) = u32x4{cm[0], cm[1], cm[2], cm[3]};
+            *reinterpret_cast<u32x4*>(p + 2 * kVPlane) = u32x4{cl[0], cl[1], cl[2], cl[3]};
+        };
+        auto k_frag = [&](int t, int plane) {  // K[key col][16t + 8hh ..]
+            return *reinterpret_cast<const u32x4*>(kpl + col * kKRowB + 16 * hh + 32 * t + plane * kKPlane);
+        };
+        auto v_frag = [&](int x, int plane) {  // step s = x/4, d = 32 (x%4) + col
+            return *reinterpret_cast<const u32x4*>(vpl + (32 * (x & 3) + col) * kVRowB + 32 * (x >> 2) + 16 * hh +
+                                                   plane * kVPlane);
         };
 
-        // S^T = K . Q^T for the K tile at Kt (padded rows); the operand of step k4+1 is
-        // read while the four MFMAs of step k4 run
-        auto qk = [&](const float* Kt, floatx16& acc) {
+        if (pass > 0) lds_barrier();  // every wave has stored its rows from the staging area
+        stage_q(u);
+        load_norm(u);
+        if (n_mine > 0) load_k(0);
+        wait_vmcnt<0>();
+        read_q();
+        if (n_mine > 0) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-            const float* kp = Kt + col * kKS_F + 4 * hh;  // K[key col][8*k4 + 4*hh ..]
-            float4 kv = *reinterpret_cast<const float4*>(kp);
+            for (int x = 0; x < 2; ++x) conv_k(x);
+            load_v(0);
+        }
+        floatx16 o[4];
+        float m, lsum;
+        auto clear = [&]() {
 #pragma unroll
-            for (int k4 = 0; k4 < 16; ++k4) {
-                const float4 kn = *reinterpret_cast<const float4*>(kp + 8 * ((k4 + 1) & 15));
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.x, qreg[4 * k4 + 0], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.y, qreg[4 * k4 + 1], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.z, qreg[4 * k4 + 2], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, qreg[4 * k4 + 3], acc, 0, 0, 0);
-                kv = kn;
-            }
+            for (int db = 0; db < 4; ++db)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) o[db][i] = 0.f;
+            m = -INFINITY;
+            lsum = 0.f;
         };
-
-        // One tile kt of this group: softmax of its scores s (in place: s becomes P^T) and
-        // O^T += V^T . P^T with V at Vt, while the scores of the K tile at Kn go to sn.  The
-        // group's last tile passes the other (stale) K buffer as Kn and discards sn: a straight-line
-        // body keeps O in 64 VGPRs (a branch around either product makes the compiler
-        // split O across register files and spill at two waves per SIMD).
-        // In-loop DMA for the next tiles: issued one or two instructions per MFMA sub-step, so
-        // their issue time hides under the matrix pipe instead of idling it.  kin / vin: a K
-        // (V) tile lies wholly below T and is fetched from scalar bases sbk / sbv into LDS at
-        // lbk / lbv (tiles reaching past T are fetched up front through the clamped path).
-        constexpr int NKI = 2 * DMA_PER_WAVE, NVI = DMA_PER_WAVE, NDI = NKI + NVI;
-        const int r0k = hw * 2 * DMA_PER_WAVE, i0v = hw * DMA_PER_WAVE;
-        auto step = [&](floatx16& s, floatx16& sn, int kt, const float* Kn, const float* Vt, bool kin, uint64_t sbk,
-                        uint32_t lbk, bool vin, uint64_t sbv, uint32_t lbv) {
+        // scores s of tile kt -> P (in place), the running maximum and sum, O rescaled if it rose
+        auto softmax = [&](int kt, floatx16& s) {
             if (kt >= nfull) {  // tile crosses the diagonal (wave-uniform)
-                const int k0 = kt * kKT + 4 * hh;
+                const int k0 = unhoisted(kt * kKT + 4 * hh);
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     if (k0 + 8 * (r >> 2) + (r & 3) > qpos) s[r] = -INFINITY;
@@ -444,7 +509,7 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
 #pragma unroll
                 for (int db = 0; db < 4; ++db)
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) o[db][i] *= corr;
+                    for (int r = 0; r < 16; ++r) o[db][r] *= corr;
                 m = mn;
             }
             const float nb_ = m == -INFINITY ? 0.f : -m;
@@ -453,145 +518,113 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
                 s[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], sl2, nb_));
                 lsum += s[r];
             }
-            // the next tile's score chain (64 dependent MFMAs) interleaved with this tile's
-            // P.V (four independent chains): one wave keeps the matrix pipe busy without
-            // waiting on its own accumulator
-            const float* vp = Vt + 4 * hh * D + 4 * col;
-            auto vrow = [&](int r) {
-                return *reinterpret_cast<const float4*>(vp + (8 * (r >> 2) + (r & 3)) * D);
-            };
+        };
+        // The same two products in fp32 from the cache (q = h + m + l is exact), for a wave whose
+        // planes gave something not finite: see after the key loop.
+        auto qk_fp32 = [&](int i, floatx16& s) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) sn[i] = 0.f;
-            const float* kp = Kn + col * kKS_F + 4 * hh;
-            float4 kv = *reinterpret_cast<const float4*>(kp);
-            float4 vv = vrow(0);
+            for (int r = 0; r < 16; ++r) s[r] = 0.f;
+            const __amdgpu_buffer_rsrc_t rs = tile_rsrc(kbase, (kt_lo + kKS * i + grp) * kKT);
+            const uint32_t off = unhoisted(col) * row_bytes + 32u * hh;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float4 kn = *reinterpret_cast<const float4*>(kp + 8 * ((r + 1) & 15));
-                const float4 vn = vrow((r + 1) & 15);
+            for (int t = 0; t < 8; ++t) {
 #pragma unroll
-                for (int x = r * NDI / 16; x < (r + 1) * NDI / 16; ++x) {
-                    if (x < NKI) {
-                        if (kin && hh == 0)  // one padded K row per instruction (lanes 0..31)
-                            dma16_s(sbk + (uint64_t)x * row_bytes, voff_k, lbk + (r0k + x) * (kKS_F * 4));
-                    } else if (vin) {  // two V rows per instruction
-                        dma16_s(sbv + (uint64_t)(2 * (x - NKI)) * row_bytes, voff_v, lbv + (i0v + x - NKI) * 1024);
-                    }
+                for (int j = 0; j < 4; ++j) {  // d = 16t + 8hh + 2j and the next
+                    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rs, off + 64 * t + 8 * j, 0, 0);
+                    const uint32_t h = unhoisted(qp[t].h[j]), m = unhoisted(qp[t].m[j]), l = unhoisted(qp[t].l[j]);
+                    const float q0 = (__uint_as_float(h << 16) + __uint_as_float(m << 16)) + __uint_as_float(l << 16);
+                    const float q1 = (__uint_as_float(h & 0xFFFF0000u) + __uint_as_float(m & 0xFFFF0000u)) +
+                                     __uint_as_float(l & 0xFFFF0000u);
+                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(v.x), q0, s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(v.y), q1, s, 0, 0, 0);
                 }
-                __builtin_amdgcn_sched_barrier(0);  // step r+1's operands are read before step r's MFMAs
-                sn = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.x, qreg[4 * r + 0], sn, 0, 0, 0);
-                o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.x, s[r], o[0], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
-                sn = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.y, qreg[4 * r + 1], sn, 0, 0, 0);
-                o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.y, s[r], o[1], 0, 0, 0);
+            }
+        };
+        auto pv_fp32 = [&](int i, const floatx16& p) {
+            const __amdgpu_buffer_rsrc_t rs = tile_rsrc(vbase, (kt_lo + kKS * i + grp) * kKT);
+            const uint32_t off = unhoisted(4 * hh) * row_bytes + 4u * col;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {  // lane half hh: key 8(r/4) + 4hh + r%4
+#pragma unroll
+                for (int db = 0; db < 4; ++db) {
+                    const float v = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                        rs, off + (8 * (r >> 2) + (r & 3)) * row_bytes + 128 * db, 0, 0));
+                    o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, p[r], o[db], 0, 0, 0);
+                }
                 __builtin_amdgcn_sched_barrier(0);
-                sn = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.z, qreg[4 * r + 2], sn, 0, 0, 0);
-                o[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.z, s[r], o[2], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-                sn = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, qreg[4 * r + 3], sn, 0, 0, 0);
-                o[3] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.w, s[r], o[3], 0, 0, 0);
-                kv = kn;
-                vv = vn;
-                __builtin_amdgcn_sched_barrier(0);  // prefetch distance stays one step (register budget)
             }
         };
 
-        // K buffers hold tiles i (even i in K0) and i+1; V buffers tile i.  At iteration
-        // i: DMA K(i+2) -> K[i%2] and V(i+1) -> V[(i+1)%2] (both last read in iteration
-        // i-1), read K(i+1) and V(i) (both landed by the wait + barrier ending i-1).
-        // The score tiles alternate between sa and sb (loop unrolled by two).
-        if (pass > 0) __syncthreads();  // every wave has stored its rows from the staging area
-        PSTAMP(1 + 5 * pass);
-        stage_q(u);
-        load_norm(u);
-        floatx16 sa, sb;
-        if constexpr (!kNormQ) {
-            // q rows and the first two K tiles are fetched together (K buffers lie outside the
-            // staging area); the first V tile, which the staging area overlaps, once q is in
-            // registers, and it lands while the first score chain runs.  (With the q norm
-            // between, the same order measured 0.5% slower than fetching the tiles after it.)
-            constexpr int kKI = 2 * DMA_PER_WAVE, kVI = DMA_PER_WAVE;  // DMA instructions per wave per K / V tile
-            if (n_mine > 0) dma_k(0, 0);
-            if (n_mine > 1) dma_k(1, 1);
-            if (n_mine > 1) wait_vmcnt<2 * kKI>();  // older than the K tiles: the q rows
-            else if (n_mine > 0) wait_vmcnt<kKI>();
-            else wait_vmcnt<0>();
-            read_q();
-            __syncthreads();  // every wave has its q: the staging area is free for the V tiles
-            if (n_mine > 0) dma_v(0, 0);
-            if (n_mine > 1) wait_vmcnt<kKI + kVI>();  // K0 has landed (K1 and V0 may fly)
-            else if (n_mine > 0) wait_vmcnt<kVI>();
-            __syncthreads();
-            if (n_mine > 0) qk(gsm, sa);
-            wait_vmcnt<0>();  // K1 and V0
-            __syncthreads();
-        } else if constexpr (kEarlyK) {
-            // the first two K tiles fly with the raw q rows and the norm's operands (K buffers lie
-            // outside the staging area): one round trip before the norm instead of two; the first V
-            // tile, which the staging area overlaps, once q is in registers, landing under the
-            // first score chain
-            if (n_mine > 0) dma_k(0, 0);
-            if (n_mine > 1) dma_k(1, 1);
-            wait_vmcnt<0>();
-            read_q();
-            __syncthreads();  // every wave has its q: the staging area is free for the V tiles
-            if (n_mine > 0) dma_v(0, 0);
-            if (n_mine > 0) qk(gsm, sa);
-            wait_vmcnt<0>();  // V0
-            __syncthreads();
-        } else {
-            wait_vmcnt<0>();
-            read_q();
-            __syncthreads();  // every wave has its q (the staging area is reused by the tile buffers)
-            if (n_mine > 0) {
-                dma_k(0, 0);
-                dma_v(0, 0);
+        clear();
+        lds_barrier();  // every wave has its q (the staging area is free for the V planes); K planes stored
+        // the groups run half an iteration apart: one multiplies K by Q while the other is in its
+        // softmax, so a SIMD's two waves do not leave the matrix pipe idle together
+        if (grp == 1) lds_barrier();
+        for (int i = 0; i < n_it; ++i) {
+            floatx16 s;
+            if (i < n_mine) {
+                // S^T = K . Q^T, while V(i) goes to its planes; then K(i+1) is fetched
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[r] = 0.f;
+                Planes kf;
+                kf.l = k_frag(0, 2), kf.m = k_frag(0, 1), kf.h = k_frag(0, 0);
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    if (t == 4 || t == 6) conv_v(t == 6);
+                    mfma_split(kf, qp[t], s, [&](int p) { return t < 7 ? k_frag(t + 1, p) : u32x4{}; });
+                }
+                if (i + 1 < n_mine) load_k(i + 1);
             }
-            if (n_mine > 1) dma_k(1, 1);
-            wait_vmcnt<0>();
-            __syncthreads();
-            if (n_mine > 0) qk(gsm, sa);
-        }
-        // paged: the cache row of the K tile fetched at iteration i + 1 is looked up at iteration
-        // i (one scalar load in flight across an MFMA stream), and the V tile fetched at i + 1 is
-        // the K tile of i, whose row is known by then; tiles past the range read no table entry
-        PSTAMP(2 + 5 * pass);
-        auto tile_row = [&](int i) -> uint32_t {  // cache row of this group's i-th tile, or 0
-            const int kt = kt_lo + kKS * i + grp;
-            return i < n_mine && (kt + 1) * kKT <= T ? crow(kt * kKT) : 0u;
-        };
-        uint32_t row_k = 0, row_v = 0;
-        if constexpr (kPaged) {
-            row_k = tile_row(2);
-            row_v = tile_row(1);
-        }
-        auto iter = [&](int i, floatx16& s, floatx16& sn) {
-            const int tk = (kt_lo + kKS * (i + 2) + grp) * kKT, tv = (kt_lo + kKS * (i + 1) + grp) * kKT;
-            const bool kdo = i + 2 < n_mine, vdo = i + 1 < n_mine;
-            const bool kin = kdo && tk + kKT <= T, vin = vdo && tv + kKT <= T;
-            if (kdo && !kin) dma_k(i + 2, i & 1);
-            if (vdo && !vin) dma_v(i + 1, (i + 1) & 1);
-            const uint32_t rk = kPaged ? row_k : (uint32_t)tk, rv = kPaged ? row_v : (uint32_t)tv;
-            if constexpr (kPaged) {
-                row_v = row_k;
-                row_k = tile_row(i + 3);
+            lds_barrier();
+            if (i < n_mine) {
+                __builtin_amdgcn_s_setprio(1);
+                softmax(kt_lo + kKS * i + grp, s);
+                // O^T += V^T . P^T, while K(i+1) goes to its planes; then V(i+1) is fetched
+                const bool more = i + 1 < n_mine;
+                Planes vf, pp;
+                vf.l = v_frag(0, 2), vf.m = v_frag(0, 1), vf.h = v_frag(0, 0);
+#pragma unroll
+                for (int x = 0; x < 8; ++x) {
+                    if ((x & 3) == 0) {
+                        uint32_t ph[4], pm[4], pl[4];
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            split_pair(s[2 * x + 2 * j], s[2 * x + 2 * j + 1], ph[j], pm[j], pl[j]);
+                        pp = {u32x4{ph[0], ph[1], ph[2], ph[3]}, u32x4{pm[0], pm[1], pm[2], pm[3]},
+                              u32x4{pl[0], pl[1], pl[2], pl[3]}};
+                    }
+                    if (x == 4 || x == 6) conv_k(x == 6);
+                    mfma_split(vf, pp, o[x & 3], [&](int p) { return x < 7 ? v_frag(x + 1, p) : u32x4{}; });
+                }
+                if (more) load_v(i + 1);
+                __builtin_amdgcn_s_setprio(0);
             }
-            const uint64_t sbk = kb_bytes + (uint64_t)(rk + r0k) * row_bytes;
-            const uint64_t sbv = vb_bytes + (uint64_t)(rv + 2 * i0v) * row_bytes;
-            const uint32_t lbk = __builtin_amdgcn_readfirstlane(lds_addr(gsm + (i & 1) * kKTileF));
-            const uint32_t lbv = __builtin_amdgcn_readfirstlane(lds_addr(gsv + ((i + 1) & 1) * kVTileF));
-            if (i < n_mine)
-                step(s, sn, kt_lo + kKS * i + grp, gsm + ((i + 1) & 1) * kKTileF, gsv + (i & 1) * kVTileF, kin, sbk,
-                     lbk, vin, sbv, lbv);
-            wait_vmcnt<0>();
-            __syncthreads();
-        };
-        for (int i = 0; i < n_it; i += 2) {
-            iter(i, sa, sb);
-            if (i + 1 < n_it) iter(i + 1, sb, sa);
+            lds_barrier();
+        }
+        if (grp == 0) lds_barrier();
+
+        // An infinite K or V value (or a finite one past bf16's range) has no planes to multiply:
+        // the residual of inf is NaN, and inf times a zero residual is NaN where the fp32 product is
+        // infinite or the key's weight is zero.  Such a tile shows as a sum that is not finite; the
+        // wave then takes its tiles again in fp32, whose outcome stands whatever it is.
+        {
+            float z = lsum * 0.f;
+#pragma unroll
+            for (int db = 0; db < 4; ++db)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) z = __builtin_fmaf(o[db][r], 0.f, z);
+            if (__builtin_amdgcn_ballot_w64(z != 0.f)) {
+                clear();
+                for (int i = 0; i < n_mine; ++i) {
+                    floatx16 s;
+                    qk_fp32(i, s);
+                    softmax(kt_lo + kKS * i + grp, s);
+                    pv_fp32(i, s);
+                }
+            }
         }
 
-        PSTAMP(3 + 5 * pass);
         // ---- merge the key groups through LDS (tile buffers are free after the barrier):
         // group g finalises output blocks db = 2g, 2g+1 and hands the other two to its partner
         float* xw = smem + w * (kXchF * 64) + lane;
@@ -605,7 +638,7 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
             xw[(2 + i) * 64] = give0[i];
             xw[(18 + i) * 64] = give1[i];
         }
-        __syncthreads();
+        lds_barrier();
         const float* xp = smem + ((1 - grp) * GW + hw) * (kXchF * 64) + lane;
         const float mp = xp[0], lp = xp[64];
         const float mt = fmaxf(m, mp);  // -inf only when this share holds no visible key for the query
@@ -616,36 +649,39 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
         // staging area in row order, then every wave stores two whole 512-byte rows per instruction
         {
             const float inv = ksplit == 1 ? 1.f / l : 1.f;
-            float* ost = qst + (hw * kQB + col) * kKS_F + 2 * grp;
+            float* ost = qst + (hw * kQB + col) * kKS_F + 64 * grp + 4 * hh;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                // O^T register r of block db is d = 4*(8(r/4) + 4hh + r%4) + db
-                float2 v;
-                v.x = (keep0[r] * c0 + xp[(2 + r) * 64] * cp) * inv;
-                v.y = (keep1[r] * c0 + xp[(18 + r) * 64] * cp) * inv;
-                *reinterpret_cast<float2*>(ost + 4 * (8 * (r >> 2) + 4 * hh + (r & 3))) = v;
+            for (int r = 0; r < 16; r += 4) {
+                // O^T registers r .. r+3 of block db are d = 32 db + 8(r/4) + 4hh + 0 .. 3
+                float v0[4], v1[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    v0[j] = (keep0[r + j] * c0 + xp[(2 + r + j) * 64] * cp) * inv;
+                    v1[j] = (keep1[r + j] * c0 + xp[(18 + r + j) * 64] * cp) * inv;
+                }
+                *reinterpret_cast<float4*>(ost + 2 * r) = make_float4(v0[0], v0[1], v0[2], v0[3]);
+                *reinterpret_cast<float4*>(ost + 32 + 2 * r) = make_float4(v1[0], v1[1], v1[2], v1[3]);
             }
             if (ksplit > 1 && live && b < B && hh == 0 && grp == 0)
                 *reinterpret_cast<float2*>(part_ml + ((size_t)split * B * H + (size_t)b * H + h) * 2) =
                     make_float2(mt, l);
         }
-        __syncthreads();
+        lds_barrier();
         {
             const int sl = kSlots * u + (wu >> 1);  // wave wu stores rows 16*(wu&1).. of slot wu/2
             const int qbo = fdiv(sl, fG), ho = kvh * G + sl - qbo * G;
             float* dst0 = ksplit == 1 ? out : part_o + (size_t)split * B * H * D;
+            const int hh0 = unhoisted(hh);
 #pragma unroll
             for (int j = 0; j < kQB / 4; ++j) {
-                const int jj = (kQB / 2) * (wu & 1) + 2 * j + hh;
+                const int jj = (kQB / 2) * (wu & 1) + 2 * j + hh0;
                 const int bo = qbo * kQB + jj;
                 const float4 v = *reinterpret_cast<const float4*>(qst + ((wu >> 1) * kQB + jj) * kKS_F + 4 * col);
                 if (sl < nslot && bo < B)
                     *reinterpret_cast<float4*>(dst0 + ((size_t)bo * H + ho) * D + 4 * col) = v;
             }
         }
-        PSTAMP(4 + 5 * pass);
     }
-    PSTAMP(11);
 }
 
 // Merge of the ksplit shares of every (query, head): grid ceil(B*H/4), 128 threads; thread
@@ -741,16 +777,15 @@ size_t prefill_ws_bytes(int B, int H, int HKV, int max_kv) {
     return align256((size_t)k * rows * kHeadDim * sizeof(float)) + align256((size_t)k * rows * 2 * sizeof(float));
 }
 
-template <bool kNormQ, bool kPaged, bool kEarlyK = false>
+template <bool kNormQ, bool kPaged>
 static hipError_t launch_prefill_kernel(hipStream_t st, unsigned grid, size_t lds, const float* q, long q_stride,
                                         float* out, const float* kc, const float* vc, const int* pos_dev, int B, int H,
                                         int HKV, float scale, int ksplit, float* part_o, float* part_ml,
                                         const float* q_gamma, const float* cs, float eps, const int* btab,
                                         int bshift, int max_blocks) {
     static std::atomic<bool> opted;
-    if (const hipError_t e = opt_in_lds(opted, (const void*)k_prefill<kNormQ, kPaged, kEarlyK>, lds); e != hipSuccess)
-        return e;
-    k_prefill<kNormQ, kPaged, kEarlyK><<<grid, 64 * kSlots * kKS, lds, st>>>(q, q_stride, out, kc, vc, pos_dev, B, H, HKV, scale,
+    if (const hipError_t e = opt_in_lds(opted, (const void*)k_prefill<kNormQ, kPaged>, lds); e != hipSuccess) return e;
+    k_prefill<kNormQ, kPaged><<<grid, 64 * kSlots * kKS, lds, st>>>(q, q_stride, out, kc, vc, pos_dev, B, H, HKV, scale,
                                                                     ksplit, part_o, part_ml, q_gamma,
                                                                     reinterpret_cast<const float2*>(cs), eps, btab,
                                                                     bshift, max_blocks);
@@ -771,19 +806,11 @@ hipError_t launch_prefill(hipStream_t st, const float* q, long q_stride, float* 
         part_ml = reinterpret_cast<float*>(static_cast<char*>(ws) + align256((size_t)ksplit * rows * kHeadDim * 4));
     }
     const size_t lds = (size_t)kLdsF * sizeof(float);  // > 64 KB: opt in once
-    static_assert(kQStageF == kVBaseF && kQStageF <= kLdsF, "merge exchange below the staging area");
     static_assert(kLdsF * sizeof(float) <= 160 * 1024, "LDS budget");
     const bool nq = q_gamma != nullptr, pg = block_table != nullptr;
     hipError_t e;
     if (nq && pg) return hipErrorInvalidValue;  // not built: a paged step norms q in its prologue
-    static const int early = [] {  // tuning aid: EI_PREFILL_EARLYK=0/1 forces the q-norm kernel's fetch order
-        const char* v = std::getenv("EI_PREFILL_EARLYK");
-        return v ? std::atoi(v) : -1;
-    }();
-    if (nq && (early == 1 || (early < 0 && ksplit > 1)))
-        e = launch_prefill_kernel<true, false, true>(st, grid, lds, q, q_stride, out, kc, vc, pos_dev, B, H, HKV,
-                                                     scale, ksplit, part_o, part_ml, q_gamma, cs, eps, nullptr, 0, 0);
-    else if (nq)
+    if (nq)
         e = launch_prefill_kernel<true, false>(st, grid, lds, q, q_stride, out, kc, vc, pos_dev, B, H, HKV, scale,
                                                ksplit, part_o, part_ml, q_gamma, cs, eps, nullptr, 0, 0);
     else if (pg)
@@ -802,9 +829,3 @@ hipError_t launch_prefill(hipStream_t st, const float* q, long q_stride, float* 
 }
 
 }  // namespace ei
-
-#ifdef EI_EXP_STAMPS
-extern "C" __attribute__((visibility("default"))) int ei_diag_prefill_stamps(void* host, size_t n) {
-    return (int)hipMemcpyFromSymbol(host, HIP_SYMBOL(ei::g_pstamps), n * 8, 0, hipMemcpyDeviceToHost);
-}
-#endif

@@ -220,8 +220,8 @@ int ei_decode_step_paged(ei_stream_t stream, const float* qkv, long row_stride, 
 /* ------------------------------------------------------------------ causal prefill
  * B query rows (row b at q + b*q_stride, heads [n_head][128], already normed + roped) at
  * positions *pos_dev + b; query b attends to cache rows 0 .. *pos_dev + b (the whole
- * chunk's K/V must already be appended).  out [B][n_head][128].  fp32 MFMA contraction
- * with online softmax.  Replaces k_attn_prefill64 (src/cuda/model_cuda.cu:1204-1341);
+ * chunk's K/V must already be appended).  out [B][n_head][128].  Matrix-core contraction of
+ * fp32 operands (three bf16 planes each, fp32 accumulate) with online softmax.  Replaces k_attn_prefill64 (src/cuda/model_cuda.cu:1204-1341);
  * the math is the CPU reference's per-token attention (src/model.cpp:138-140, :191-214). */
 int ei_attn_prefill(ei_stream_t stream, const float* q, long q_stride, float* out, const float* kc, const float* vc,
                     const int* pos_dev, int B, int n_head, int n_head_kv, int head_dim, float scale);

@@ -1,0 +1,95 @@
+"""GPU tests of the prefill kernel's three-plane products: every fp32 K, V, Q and P value is
+multiplied as three bf16 planes that together hold all its bits.  Sizes sit at the edges of the
+tiles (32 keys, 32-query blocks, units of 4 slots, two key groups), values at the edges of the
+planes' range."""
+import numpy as np
+import pytest
+
+from tests.parity import ATTN_RTOL, rel_err
+
+pytestmark = pytest.mark.gpu
+
+D = 128
+
+
+def _run(gpu, q, k, v, pos0, H, HKV, ws=None):
+    import torch
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, k, v)]
+    pos = torch.tensor([pos0], dtype=torch.int32, device="cuda")
+    out = gpu.attn_prefill(dev[0], dev[1], dev[2], pos, gpu.AttnShape(H, HKV), ws=ws)
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+def _exact(q, k, v, pos0, H, HKV, dtype=np.float64):
+    B, G = q.shape[0], H // HKV
+    qd, kd, vd = (x.astype(dtype) for x in (q.reshape(B, H, D), k, v))
+    out = np.zeros((B, H, D), dtype)
+    for b in range(B):
+        T = pos0 + b + 1
+        for h in range(H):
+            s = kd[:T, h // G] @ qd[b, h] / np.sqrt(dtype(D))
+            p = np.exp(s - s.max())
+            out[b, h] = (p / p.sum()) @ vd[:T, h // G]
+    return out
+
+
+def _inputs(orc, B, pos0, H, HKV, seed):
+    n = pos0 + B
+    return (orc.normal((B, H * D), seed), orc.normal((n, HKV, D), seed + 1), orc.normal((n, HKV, D), seed + 2))
+
+
+def _close(got, exact):
+    """Single elements within the attention bar, and the 2-norm within 1e-6.  An fp32 score of |s| ~ 11
+    over 48 roundings is off by ~1.2e-7 (times the softmax scale), the exponent's argument and the
+    exponential by ~1e-7 each, the value sums by less: 2e-7 to 5e-7 together.  A second-order plane
+    product left out (2^-18 of |q||k|) alone is 1.3e-6."""
+    off = np.linalg.norm(got.astype(np.float64) - exact) / np.linalg.norm(exact)
+    assert off <= 1e-6, off
+    assert rel_err(got, exact) <= ATTN_RTOL
+
+
+@pytest.mark.parametrize("H,HKV,B,pos0", [(4, 1, 1, 0), (4, 1, 31, 0), (4, 1, 33, 31), (8, 2, 32, 32), (8, 2, 65, 63),
+                                          (8, 1, 40, 29), (5, 1, 97, 1), (2, 2, 129, 64), (6, 2, 64, 95),
+                                          (4, 1, 16, 1000)])
+def test_prefill_error_against_float64(orc, gpu, H, HKV, B, pos0):
+    q, k, v = _inputs(orc, B, pos0, H, HKV, 31000 + B + pos0)
+    exact = _exact(q, k, v, pos0, H, HKV)
+    for ws in (None, gpu.PrefillWorkspace(B, H, HKV, max(pos0 + B, 4096))):
+        got = _run(gpu, q, k, v, pos0, H, HKV, ws)
+        _close(got, exact)
+
+
+def test_prefill_small_and_large_magnitudes(orc, gpu):
+    """Planes keep fp32's exponent range: values near 1e-33 keep all their bits, and K near the
+    largest float against tiny q gives ordinary scores.  Same bound as above."""
+    H, HKV, B, pos0 = 4, 1, 40, 50
+    q, k, v = _inputs(orc, B, pos0, H, HKV, 32000)
+    got = _run(gpu, q * np.float32(2.0 ** -100), k * np.float32(2.0 ** 100), v * np.float32(2.0 ** -110), pos0, H, HKV)
+    exact = _exact(q, k, v, pos0, H, HKV)
+    _close(got.astype(np.float64) * 2.0 ** 110, exact)
+
+
+@pytest.mark.parametrize("split", [False, True])
+def test_prefill_infinite_and_huge_values(orc, gpu, split):
+    """An infinite K element whose scores are -inf drops the key and leaves finite rows; a V element
+    past bf16's largest value stays the finite number it is; an infinite V element gives an infinite
+    output in its own column only; a NaN in V stays in its column."""
+    H, HKV, B, pos0 = 4, 1, 70, 60
+    q, k, v = _inputs(orc, B, pos0, H, HKV, 33000)
+    ws = gpu.PrefillWorkspace(B, H, HKV, 4096) if split else None
+    q[:, ::D] = np.abs(q[:, ::D]) + np.float32(0.1)  # element 0 of every head positive
+    k[37, 0, 0] = -np.inf
+    ref = _exact(q, k, v, pos0, H, HKV)
+    assert np.isfinite(ref).all()
+    _close(_run(gpu, q, k, v, pos0, H, HKV, ws), ref)
+    v[5, 0, 9] = np.float32(3.4e38)
+    v[11, 0, 17] = np.inf
+    v[12, 0, 21] = np.nan
+    with np.errstate(invalid="ignore"):
+        ref = _exact(q, k, v, pos0, H, HKV)
+    got = _run(gpu, q, k, v, pos0, H, HKV, ws)
+    assert np.isposinf(got[..., 17]).all() and np.isnan(got[..., 21]).all()
+    cols = [c for c in range(D) if c not in (9, 17, 21)]
+    _close(got[..., cols], ref[..., cols])
+    assert np.max(np.abs(got[..., 9] / ref[..., 9] - 1.0)) <= 1e-5  # one term rules the column: p's own error
