@@ -240,13 +240,6 @@ __device__ __forceinline__ int unhoisted(int x) {
     return x;
 }
 
-// Workgroup barrier ordering LDS only: global loads stay in flight across it.
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // kPaged: key t of the sequence sits in pool row btab[t >> bshift] << bshift | (t & mask), the
 // block size 2^bshift >= 32, so a 32-key tile lies in one block and its rows are consecutive.
 template <bool kNormQ, bool kPaged>

@@ -8,35 +8,44 @@
 // RoPE and the cache append that the reference launches next (three more kernels) are the
 // epilogue that ei_decode_step / ei_decode_step_paged apply inside the attention launch.
 //
-// A decode step's projection is bound by the weight stream (E x (H + 2 HKV) x 128 weights read
-// once per token: 63 MB in fp32, 31 MB in fp16 at Qwen3-4B), so the kernel is a streaming
-// GEMV: wave w of a workgroup owns kRowsPerWave consecutive output rows; lane l reads 16-byte
-// pieces l, l + 64, ... of each row (whole 1 KB per instruction, non-temporal: read once),
-// issues every piece of its rows before any arithmetic, and only then stages the normed
-// activations: the x rows are read (L2-resident after the first workgroups), their sum of
-// squares is taken in double as the CPU rmsnorm does, and h = (x * inv) * gamma goes to LDS,
-// read back as broadcast 16-byte pieces.  Dot products accumulate per lane with FMAs and end
-// in a wave butterfly; up to kMaxRows activation rows share each weight load.
+// A decode step's projection streams the weights once per launch (E x (H + 2 HKV) x 128 weights:
+// 63 MB in fp32, 31 MB in fp16, 9-17 MB in blocks at Qwen3-4B).  One workgroup per CU keeps to a
+// contiguous range of output rows.  A row's E weights are spread over the lanes of a row group (L lanes,
+// 8 to 32 weights each; 1 to 8 groups to a workgroup work on different rows), so the normed activations
+// that a lane multiplies by are the same for every row: they are loaded, normed and kept in registers
+// once, and nothing but weights moves after that.  (Read from LDS for every pair of rows, as this kernel
+// did before, they were the bound with several activation rows: each wave read rows x E x 4 bytes for
+// two weight rows, and waited for every read by itself.)  A lane keeps RB rows of weights in flight:
+// each row's registers are loaded again, with the row RB further on, as soon as they are used, so the
+// stream runs on under the arithmetic.  The partial sums of RB rows x NB activation rows are added over
+// 32 lanes by one transposing butterfly and over the half-waves of the group through LDS.
+//
+// Measured, graph-timed per launch, before -> now (us; a plain read of the weights takes 6.2 at 31.5 MB, 8.7 at
+// 50 MB): F16 at E 2560, 6144 outputs, 2 rows 12.6 -> 8.3, 4 rows 24.3 -> 9.9; E 4096, 4 rows 39.4 -> 12.1; E 5120,
+// 7168 outputs, 4 rows 75.3 -> 17.1; F32 there 66.6 -> 26.1; Q8_0 41.3 -> 16.4; Q4_K 40.1 -> 15.5; Q6_K 48.6 ->
+// 17.1; one row of Q6_K at 5120 18.7 -> 15.8; Q4_K at E 1024, 4096 outputs, 4 rows 5.9 -> 4.5.  Several rows cost
+// little more than one now: the stream bounds them, and what is left over it is the launch's start, the norm
+// and the last batch's sums.  Tried and not kept: the sums in LDS-read order with four or eight waves a
+// workgroup (F16, E 2560, 4 rows: 14.2), activations loaded lane by lane from memory (16 values a lane, 64
+// bytes apart: Q4_K one row 7.3 against 6.4), two workgroups a CU (8.9), 15 waves (7.8), branches around the
+// reloads (vmcnt waits for everything behind them; F32 one row 15.0 against 11.6).
 //
 // Quantised weights (Q8_0, Q4_K, Q6_K: the block formats the reference computes with,
 // src/quant.h:21-39) stay in their GGUF block layout.  Each lane decodes items of 16
 // consecutive values (half a Q8_0 block, half a 32-value Q4_K sub-block, a 16-value Q6_K group)
-// of one of its wave's two rows, with the reference's values (src/quant.cpp:7-60), so every
+// straight from registers, with the reference's values (src/quant.cpp:7-60), so every
 // weight is the float the CPU path's convert_row gives, before the same FMA dot as the float
-// kernels.  Q4_K blocks are whole 16-byte pieces, so each lane loads the two pieces an item needs
-// straight into registers; Q8_0 and Q6_K rows are loaded as coalesced pieces (16-byte, or 4-byte
-// for Q6_K) and parked in a wave-private LDS area first.
+// kernels.
 #include <hip/hip_fp16.h>
+
+#include <type_traits>
 
 #include "common.h"
 #include "launch.h"
 
 namespace ei {
 
-constexpr int kProjWaves = 4;
-constexpr int kRowsPerWave = 2;
-constexpr int kProjMaxLdsFloats = 24576;  // B * E activations staged in LDS (96 KB)
-
+constexpr int kProjMaxLdsFloats = 24576;  // rows per launch at hidden size E: at most this over E
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ void f16x8(const u32x4_t u, float* f) {
@@ -49,115 +58,7 @@ __device__ __forceinline__ void f16x8(const u32x4_t u, float* f) {
     }
 }
 
-// WF16: weights are binary16; NB activation rows (B <= NB); P 16-byte pieces per lane per row,
-// E = 64 * P * (4 fp32 or 8 fp16 weights per piece), fixed at compile time so the weights stay
-// in registers
-template <bool WF16, int NB, int P>
-__global__ __launch_bounds__(64 * kProjWaves) void k_qkv_project(const float* __restrict__ x, long x_stride, int B,
-                                                                 int E, const float* __restrict__ gamma, float eps,
-                                                                 const void* __restrict__ w, int n_out,
-                                                                 float* __restrict__ out, long out_stride) {
-    constexpr int kPer = WF16 ? 8 : 4;  // weights per 16-byte piece
-    extern __shared__ __align__(16) float hs[];  // [NB][E] normed activations
-    __shared__ double ssum[kProjWaves][NB];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int r0 = (blockIdx.x * kProjWaves + wv) * kRowsPerWave;
-
-    // ---- this thread's activation and gamma elements first (L2-resident after the first
-    // workgroups), then every weight piece of the wave's rows: loads return in order, so the
-    // norm below waits for the activations only and overlaps the weight stream
-    constexpr int kEl = 64 * P * kPer / (64 * kProjWaves);  // elements per thread per row
-    float xv[NB][kEl], gv[kEl];
-#pragma unroll
-    for (int i = 0; i < kEl; ++i) gv[i] = gamma[tid + i * 64 * kProjWaves];
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int i = 0; i < kEl; ++i) xv[b][i] = b < B ? x[(size_t)b * x_stride + tid + i * 64 * kProjWaves] : 0.f;
-    u32x4_t wr[kRowsPerWave][P];
-#pragma unroll
-    for (int rr = 0; rr < kRowsPerWave; ++rr) {
-        const int r = min(r0 + rr, n_out - 1);
-        const char* row = static_cast<const char*>(w) + (size_t)r * E * (WF16 ? 2 : 4);
-#pragma unroll
-        for (int p = 0; p < P; ++p)
-            wr[rr][p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(row) + p * 64 + lane);
-    }
-
-    // ---- attention RMSNorm of the B rows into LDS (src/ops.cpp:155-160: sum of squares in
-    // double, inv = float(1 / sqrt(ss / E + eps)), h = (x * inv) * gamma)
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        double ss = 0.0;
-#pragma unroll
-        for (int i = 0; i < kEl; ++i) ss += (double)xv[b][i] * (double)xv[b][i];
-        ss = wave_sum_f64(ss);
-        if (lane == 0) ssum[wv][b] = ss;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        if (b >= B) break;
-        double ss = 0.0;
-#pragma unroll
-        for (int k = 0; k < kProjWaves; ++k) ss += ssum[k][b];
-        const float inv = (float)(1.0 / sqrt(ss / (double)E + (double)eps));
-#pragma unroll
-        for (int i = 0; i < kEl; ++i) {
-#pragma clang fp contract(off)
-            hs[b * E + tid + i * 64 * kProjWaves] = (xv[b][i] * inv) * gv[i];
-        }
-    }
-    __syncthreads();
-
-    // ---- dot products: lane l covers pieces p*64 + l of each row
-    float acc[kRowsPerWave][NB];
-#pragma unroll
-    for (int rr = 0; rr < kRowsPerWave; ++rr)
-#pragma unroll
-        for (int b = 0; b < NB; ++b) acc[rr][b] = 0.f;
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-        const int e0 = (p * 64 + lane) * kPer;
-#pragma unroll
-        for (int rr = 0; rr < kRowsPerWave; ++rr) {
-            float wf[kPer];
-            if constexpr (WF16) {
-                f16x8(wr[rr][p], wf);
-            } else {
-                wf[0] = __uint_as_float(wr[rr][p].x);
-                wf[1] = __uint_as_float(wr[rr][p].y);
-                wf[2] = __uint_as_float(wr[rr][p].z);
-                wf[3] = __uint_as_float(wr[rr][p].w);
-            }
-#pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                if (b >= B) break;
-#pragma unroll
-                for (int k = 0; k < kPer; k += 4) {
-                    const float4 h4 = *reinterpret_cast<const float4*>(hs + b * E + e0 + k);
-                    acc[rr][b] = fmaf(wf[k], h4.x, acc[rr][b]);
-                    acc[rr][b] = fmaf(wf[k + 1], h4.y, acc[rr][b]);
-                    acc[rr][b] = fmaf(wf[k + 2], h4.z, acc[rr][b]);
-                    acc[rr][b] = fmaf(wf[k + 3], h4.w, acc[rr][b]);
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int rr = 0; rr < kRowsPerWave; ++rr)
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            if (b >= B) break;
-            const float s = wave_sum(acc[rr][b]);
-            if (lane == 0 && r0 + rr < n_out) out[(size_t)b * out_stride + r0 + rr] = s;
-        }
-}
-
 // ------------------------------------------------------------------ quantised weights
-constexpr int kQWaves = 4;     // waves per workgroup
-constexpr int kQRowsPerWave = 2;
-
 template <int T>
 struct QFormat;
 template <>
@@ -176,13 +77,11 @@ struct QFormat<14> {  // Q6_K
 __device__ __forceinline__ float f16_bits(uint32_t h) {
     return __half2float(__ushort_as_half((unsigned short)(h & 0xFFFFu)));
 }
-__device__ __forceinline__ uint32_t lds_u16(const uint8_t* p) { return *reinterpret_cast<const uint16_t*>(p); }
-// 16 bytes from an LDS address that may be only 2-byte aligned (gfx950 LDS reads need no
-// natural alignment; memcpy lets the compiler pick the widest reads)
-__device__ __forceinline__ u32x4_t lds_16bytes(const uint8_t* p) {
-    u32x4_t v;
-    __builtin_memcpy(&v, p, 16);
-    return v;
+// 16 bytes from an address that may be only 2-byte aligned (Q8_0 and Q6_K blocks are 34 and 210
+// bytes; gfx950 global loads need no natural alignment)
+__device__ __forceinline__ u32x4_t load16(const uint8_t* p) {
+    typedef u32x4_t __attribute__((aligned(2))) u32x4_u;
+    return __builtin_nontemporal_load(reinterpret_cast<const u32x4_u*>(p));
 }
 // byte k of a word as a float (one v_cvt_f32_ubyte)
 __device__ __forceinline__ float ubyte_f(uint32_t u, int k) { return (float)((u >> (8 * k)) & 0xFFu); }
@@ -194,17 +93,66 @@ __device__ __forceinline__ uint32_t opaque(uint32_t u) {
     return u;
 }
 
-// Item k (values 16 k .. 16 k + 15) of a row whose bytes start at `row` (LDS) -> wv[16]: half
-// a Q8_0 block, half a 32-value Q4_K sub-block, or a 16-value Q6_K group with one scale.  Every
-// value is the float the reference's decode gives; the byte-wise conversions are exact.
-template <int T>
-__device__ __forceinline__ void decode16(const uint8_t* row, int k, float* wv) {
+// One row's weights of a lane, as loaded: load() from the row's first byte, values() their floats.
+// lane_in_row 0 .. L-1; F32 and F16 lanes take the 16-byte pieces c * L + lane_in_row (whole 1 KB per
+// instruction), quantised lanes item lane_in_row (values 16 lane_in_row .. + 15).
+template <int T, int E>
+struct RowShape {
+    static constexpr int kPer = T == 0 ? 4 : T == 1 ? 8 : 16;  // values per piece or item
+    // 8 values a lane (F32, F16) while a row then takes at most 512 lanes, else 16 or 32
+    static constexpr int kVals = T > 1 ? 16 : E / 8 <= 512 ? 8 : E / 16 <= 512 ? 16 : 32;
+    static constexpr int kLanes = E / kVals;  // lanes of a row group
+    static constexpr int kPieces = kVals / kPer;
+    // row groups of a workgroup: 8 waves, or 10 where a row takes 160 or 320 lanes
+    static constexpr int kGroups = kLanes == 160 ? 4 : kLanes == 320 ? 2 : 512 / kLanes;
+    static constexpr int kThreads = kLanes * kGroups;
+    static_assert(kLanes * kVals == E && kLanes % 32 == 0 && kThreads % 64 == 0 && kThreads <= 640, "hidden size");
+    // where 4 values from value e on sit in a normed activation row in LDS: the first quarters of all
+    // pieces, then the second ones, ..., so that a wave reads contiguous 16-byte parts, the rows of
+    // quarters offset against each other so that its stores spread over the banks too
+    static constexpr int kQuarters = kPer / 4, kQRow = E / kPer + (kQuarters == 4 ? 2 : kQuarters == 2 ? 4 : 0);
+    static constexpr int kHRow = 4 * kQuarters * kQRow;  // floats of a row
+    static __device__ __forceinline__ int h_at(int e) { return 4 * ((e / 4) % kQuarters * kQRow + e / kPer); }
+    // first value of piece c of a lane
+    static __device__ __forceinline__ int first(int c, int li) { return (c * kLanes + li) * kPer; }
+};
+template <int T, int E>
+struct Weights {
+    using S = RowShape<T, E>;
+    static constexpr size_t kRowBytes = (size_t)E * (T == 0 ? 4 : 2);
+    u32x4_t p[S::kPieces];
+    __device__ __forceinline__ void load(const uint8_t* row, int li) {
+#pragma unroll
+        for (int c = 0; c < S::kPieces; ++c)
+            p[c] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(row) + c * S::kLanes + li);
+    }
+    __device__ __forceinline__ void values(int, float* f) const {
+#pragma unroll
+        for (int c = 0; c < S::kPieces; ++c) {
+            if constexpr (T == 1) {
+                f16x8(p[c], f + 8 * c);
+            } else {
+                f[4 * c] = __uint_as_float(p[c].x), f[4 * c + 1] = __uint_as_float(p[c].y);
+                f[4 * c + 2] = __uint_as_float(p[c].z), f[4 * c + 3] = __uint_as_float(p[c].w);
+            }
+        }
+    }
+};
+
+template <int E>
+struct Weights<8, E> {  // Q8_0: y = q * d (src/quant.cpp:7-13); item: half a block
+    static constexpr size_t kRowBytes = (size_t)E / QFormat<8>::kValues * QFormat<8>::kBytes;
+    u32x4_t q;
+    uint32_t d16;
+    __device__ __forceinline__ void load(const uint8_t* row, int li) {
+        const uint8_t* blk = row + 34 * (li >> 1);
+        q = load16(blk + 2 + 16 * (li & 1));
+        d16 = *reinterpret_cast<const uint16_t*>(blk);
+    }
+    __device__ __forceinline__ void values(int, float* wv) const {
 #pragma clang fp contract(off)
-    if constexpr (T == 8) {  // Q8_0: y = q * d (src/quant.cpp:7-13)
-        const uint8_t* blk = row + 34 * (k >> 1);
-        const float d = f16_bits(lds_u16(blk));
+        const float d = f16_bits(d16);
         const float off = -128.f * d;  // exact (a power-of-two scaling)
-        const u32x4_t q = lds_16bytes(blk + 2 + 16 * (k & 1));
         const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -215,42 +163,60 @@ __device__ __forceinline__ void decode16(const uint8_t* row, int k, float* wv) {
 #pragma unroll
             for (int b = 0; b < 4; ++b) wv[4 * i + b] = __builtin_fmaf(ubyte_f(u, b), d, off);
         }
-    } else if constexpr (T == 12) {  // Q4_K: y = (d sc) q - dmin m (src/quant.cpp:15-33)
-        const uint8_t* blk = row + 144 * (k >> 4);
-        const int v = (k & 15) * 16, c = v >> 6, hi4 = (v >> 5) & 1, l = v & 31;
-        const uint32_t dd = *reinterpret_cast<const uint32_t*>(blk);  // d, dmin (16-byte aligned block)
-        const float d = f16_bits(dd), dmin = f16_bits(dd >> 16);
-        const uint32_t* pk = reinterpret_cast<const uint32_t*>(blk + 4);  // 12 packed bytes
-        const uint32_t p0 = pk[0], p1 = pk[1], p2 = pk[2];
-        auto pb = [&](int n) -> int { return (int)(((n < 4 ? p0 : n < 8 ? p1 : p2) >> (8 * (n & 3))) & 0xFFu); };
-        const int j = 2 * c + hi4;  // sub-block: 6-bit scale and min (src/quant.h:43-52)
-        int sc, m;
-        if (j < 4) {
-            sc = pb(j) & 63;
-            m = pb(j + 4) & 63;
-        } else {
-            sc = (pb(j + 4) & 15) | ((pb(j - 4) >> 6) << 4);
-            m = (pb(j + 4) >> 4) | ((pb(j) >> 6) << 4);
-        }
+    }
+};
+
+template <int E>
+struct Weights<12, E> {  // Q4_K: y = (d sc) q - dmin m (src/quant.cpp:15-33); item: half a 32-value sub-block
+    static constexpr size_t kRowBytes = (size_t)E / QFormat<12>::kValues * QFormat<12>::kBytes;
+    u32x4_t hdr, q;  // the block's first 16 bytes (d, dmin, 12 scale bytes); the item's nibbles
+    __device__ __forceinline__ void load(const uint8_t* row, int li) {
+        const int v = (li & 15) * 16;
+        const uint8_t* blk = row + 144 * (li >> 4);  // blocks are whole 16-byte pieces
+        hdr = *reinterpret_cast<const u32x4_t*>(blk);
+        q = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(blk + 16 + 32 * (v >> 6) + (v & 31)));
+    }
+    __device__ __forceinline__ void values(int li, float* wv) const {
+#pragma clang fp contract(off)
+        const int j = (li & 15) >> 1, hi4 = j & 1;  // sub-block: its 6-bit scale and min (src/quant.h:43-52)
+        const float d = f16_bits(hdr.x), dmin = f16_bits(hdr.x >> 16);
+        // bytes j%4 of the three words: sub-blocks 0..3 hold theirs in the low six bits of the first two,
+        // 4..7 in the nibbles of the third and the top bits of the first two
+        const uint32_t a = hdr.y >> (8 * (j & 3)), b = hdr.z >> (8 * (j & 3)), c = hdr.w >> (8 * (j & 3));
+        const uint32_t sc = j < 4 ? a & 63u : (c & 15u) | ((a >> 2) & 0x30u);
+        const uint32_t m = j < 4 ? b & 63u : ((c >> 4) & 15u) | ((b >> 2) & 0x30u);
         const float dl = d * (float)sc, ml = dmin * (float)m;
-        const u32x4_t q = *reinterpret_cast<const u32x4_t*>(blk + 16 + 32 * c + l);  // 16-byte aligned
         const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const uint32_t nib = opaque((qw[i] >> (4 * hi4)) & 0x0F0F0F0Fu);
             // dl * q is exact (17 x 4 significant bits), so the FMA rounds like dl * q - ml
 #pragma unroll
-            for (int b = 0; b < 4; ++b) wv[4 * i + b] = __builtin_fmaf(dl, ubyte_f(nib, b), -ml);
+            for (int k = 0; k < 4; ++k) wv[4 * i + k] = __builtin_fmaf(dl, ubyte_f(nib, k), -ml);
         }
-    } else {  // Q6_K: y = (d sc) (q - 32) (src/quant.cpp:35-60)
-        const uint8_t* blk = row + 210 * (k >> 4);
-        const int v = (k & 15) * 16, h = v >> 7, g = (v >> 5) & 3, l = v & 31;
-        const float d = f16_bits(lds_u16(blk + 208));
-        const float dsc = d * (float)(int8_t)blk[192 + 8 * h + (l >> 4) + 2 * g];
+    }
+};
+
+template <int E>
+struct Weights<14, E> {  // Q6_K: y = (d sc) (q - 32) (src/quant.cpp:35-60); item: a 16-value group, one scale
+    static constexpr size_t kRowBytes = (size_t)E / QFormat<14>::kValues * QFormat<14>::kBytes;
+    u32x4_t ql, qh;
+    uint32_t d16;
+    int sc;
+    __device__ __forceinline__ void load(const uint8_t* row, int li) {
+        const uint8_t* blk = row + 210 * (li >> 4);
+        const int v = (li & 15) * 16, h = v >> 7, g = (v >> 5) & 3, l = v & 31;
+        ql = load16(blk + 64 * h + l + 32 * (g & 1));
+        qh = load16(blk + 128 + 32 * h + l);
+        sc = (int8_t)blk[192 + 8 * h + (l >> 4) + 2 * g];
+        d16 = *reinterpret_cast<const uint16_t*>(blk + 208);
+    }
+    __device__ __forceinline__ void values(int li, float* wv) const {
+#pragma clang fp contract(off)
+        const int g = ((li & 15) >> 1) & 3;
+        const float dsc = f16_bits(d16) * (float)sc;
         // dsc q - 32 dsc in one rounding (32 dsc is exact): the correctly rounded dsc (q - 32)
         const float off = -32.f * dsc;
-        const u32x4_t ql = lds_16bytes(blk + 64 * h + l + 32 * (g & 1));
-        const u32x4_t qh = lds_16bytes(blk + 128 + 32 * h + l);
         const uint32_t lw[4] = {ql.x, ql.y, ql.z, ql.w}, hw[4] = {qh.x, qh.y, qh.z, qh.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -260,218 +226,337 @@ __device__ __forceinline__ void decode16(const uint8_t* row, int k, float* wv) {
             for (int b = 0; b < 4; ++b) wv[4 * i + b] = __builtin_fmaf(dsc, ubyte_f(q6, b), off);
         }
     }
+};
+
+// Sums of N values over the 32 lanes of each half-wave by a transposing butterfly: at each step a lane
+// keeps half of its values and adds its partner's copy of that half, so N values take about N exchanges
+// instead of 5 N.  v[k], k < n, of a lane then holds the sum of value at + k.
+template <int M, int N>
+__device__ __forceinline__ void half_wave_sums(float* v, int lane, int& at, int& n) {
+    if constexpr (M >= 1) {
+        constexpr int K = (N + 1) / 2;
+        const bool up = (lane & M) != 0;
+        if constexpr (N > 1) {
+#pragma unroll
+            for (int i = 0; i < K; ++i) {
+                const float hi = i + K < N ? v[i + K] : 0.f;
+                const float send = up ? v[i] : hi, keep = up ? hi : v[i];
+                v[i] = keep + lane_xor<M>(send);
+            }
+            at += up ? K : 0;
+            n = up ? n - K : min(n, K);
+        } else {
+            v[0] += lane_xor<M>(v[0]);
+        }
+        half_wave_sums<M / 2, K>(v, lane, at, n);
+    }
 }
 
-// Q4_K item from registers: hdr = the block's first 16 bytes (d, dmin, 12 scale bytes), q = the
-// item's 16 bytes of nibbles; sub-block sbj, nibble hi4.  Same arithmetic as decode16<12>.
-__device__ __forceinline__ void decode16_q4k_regs(u32x4_t hdr, u32x4_t q, int sbj, int hi4, float* wv) {
+// T the GGML weight type, NB activation rows, hidden size E, RB weight rows of a group in flight.
+// Workgroup i takes output rows [i * rows, (i + 1) * rows): group g the rows g, g + kGroups, ... of it,
+// RB at a time.
+template <int T, int NB, int E, int RB>
+__global__ __launch_bounds__((RowShape<T, E>::kThreads)) void k_qkv_project(const float* __restrict__ x, long x_stride,
+                                                                           const float* __restrict__ gamma, float eps,
+                                                                           const uint8_t* __restrict__ w, int n_out,
+                                                                           int rows, float* __restrict__ out,
+                                                                           long out_stride) {
+    using S = RowShape<T, E>;
+    using W = Weights<T, E>;
+    constexpr int NV = S::kVals, HW = S::kLanes / 32, N = RB * NB;  // HW half-waves to a row group
+    extern __shared__ __align__(16) float hs[];  // [NB][kHRow] normed activations
+    __shared__ double ssum[S::kThreads / 64][NB];
+    __shared__ float red[2][S::kThreads / 32][N];
+    const int tid = threadIdx.x, lane = tid & 63, hwave = tid >> 5, wave = tid >> 6;
+    const int grp = tid / S::kLanes, li = tid - grp * S::kLanes;
+    const int row_lo = blockIdx.x * rows, row_hi = min(row_lo + rows, n_out);
+
+    // ---- the activations and gammas first, 4 to a thread at a time, then RB rows of weights: loads return
+    // in order, so the norm waits for the activations only and runs while the weights are on their way
+    constexpr int kX = (E / 4 + S::kThreads - 1) / S::kThreads;
+    float4 xv[NB][kX], gv[kX];
+#pragma unroll
+    for (int i = 0; i < kX; ++i) {
+        const int e = 4 * min(tid + i * S::kThreads, E / 4 - 1);
+        gv[i] = *reinterpret_cast<const float4*>(gamma + e);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) xv[b][i] = *reinterpret_cast<const float4*>(x + (size_t)b * x_stride + e);
+    }
+    W wt[RB];
+    // the row of this group's j-th turn; past the range the last row again (loaded, not used)
+    auto row_at = [&](int j) { return min(row_lo + grp + j * S::kGroups, row_hi - 1); };
+#pragma unroll
+    for (int i = 0; i < RB; ++i) wt[i].load(w + (size_t)row_at(i) * W::kRowBytes, li);
+
+    // ---- attention RMSNorm (src/ops.cpp:155-160: sum of squares in double,
+    // inv = float(1 / sqrt(ss / E + eps)), h = (x * inv) * gamma)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        double ss = 0.0;
+#pragma unroll
+        for (int i = 0; i < kX; ++i) {
+            const float4 v = xv[b][i];
+            if (tid + i * S::kThreads < E / 4)
+                ss += ((double)v.x * (double)v.x + (double)v.y * (double)v.y) +
+                      ((double)v.z * (double)v.z + (double)v.w * (double)v.w);
+        }
+        ss = wave_sum_f64(ss);
+        if (lane == 0) ssum[wave][b] = ss;
+    }
+    lds_barrier();
+    {
+        // lane b of every four takes the root of activation row b
+        const int mb = NB == 1 ? 0 : min(lane & 3, NB - 1);
+        double ss = 0.0;
+#pragma unroll
+        for (int k = 0; k < S::kThreads / 64; ++k) ss += ssum[k][mb];
+        const float inv = (float)(1.0 / sqrt(ss / (double)E + (double)eps));
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const float ib = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inv), b));
+#pragma unroll
+            for (int i = 0; i < kX; ++i) {
 #pragma clang fp contract(off)
-    const float d = f16_bits(hdr.x), dmin = f16_bits(hdr.x >> 16);
-    const uint32_t p0 = hdr.y, p1 = hdr.z, p2 = hdr.w;
-    auto pb = [&](int n) -> int { return (int)(((n < 4 ? p0 : n < 8 ? p1 : p2) >> (8 * (n & 3))) & 0xFFu); };
-    int sc, m;
-    if (sbj < 4) {
-        sc = pb(sbj) & 63;
-        m = pb(sbj + 4) & 63;
-    } else {
-        sc = (pb(sbj + 4) & 15) | ((pb(sbj - 4) >> 6) << 4);
-        m = (pb(sbj + 4) >> 4) | ((pb(sbj) >> 6) << 4);
+                const float4 v = xv[b][i], g = gv[i];
+                const int e = 4 * (tid + i * S::kThreads);
+                if (e < E)
+                    *reinterpret_cast<float4*>(hs + b * S::kHRow + S::h_at(e)) =
+                        make_float4((v.x * ib) * g.x, (v.y * ib) * g.y, (v.z * ib) * g.z, (v.w * ib) * g.w);
+            }
+        }
     }
-    const float dl = d * (float)sc, ml = dmin * (float)m;
-    const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t nib = opaque((qw[i] >> (4 * hi4)) & 0x0F0F0F0Fu);
-#pragma unroll
-        for (int b = 0; b < 4; ++b) wv[4 * i + b] = __builtin_fmaf(dl, ubyte_f(nib, b), -ml);
-    }
-}
-
-// Quantised rows: T the GGML type (8, 12, 14), NB activation rows (B <= NB), hidden size E
-// (compile time: the activation, gamma and weight loads are all issued before any is used,
-// activations first, so the norm waits for them alone and overlaps the weight stream).  Row
-// bytes RB; wave w owns rows r0, r0 + 1 (clamped to the last row), their bytes at LDS
-// qrow + w * 2 RB.
-template <int T, int NB, int E>
-__global__ __launch_bounds__(64 * kQWaves) void k_qkv_project_q(const float* __restrict__ x, long x_stride, int B,
-                                                                const float* __restrict__ gamma, float eps,
-                                                                const uint8_t* __restrict__ w, int n_out,
-                                                                float* __restrict__ out, long out_stride) {
-    using F = QFormat<T>;
-    constexpr int RB = E / F::kValues * F::kBytes;
-    // Q8_0 and Q4_K rows of a multiple of 512 values are whole 16-byte pieces; Q6_K rows
-    // (210-byte blocks) are read in 4-byte pieces
-    constexpr bool wide = RB % 16 == 0;
-    constexpr int kPiece = wide ? 16 : 4;
-    constexpr int kPer = (RB / kPiece + 63) / 64;  // pieces per lane per row
-    constexpr int kEl = E / (64 * kQWaves);        // activation elements per thread per row
-    static_assert(E % (64 * kQWaves) == 0 && E % 512 == 0 && RB % 4 == 0, "hidden size");
-    extern __shared__ __align__(16) float hs[];  // [B][E] normed activations, then the rows' bytes
-    __shared__ double ssum[kQWaves][NB];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int r0 = (blockIdx.x * kQWaves + wv) * kQRowsPerWave;
-
-    // ---- activations and gamma, then this wave's row bytes (read once: non-temporal)
-    float xv[NB][kEl], gv[kEl];
-#pragma unroll
-    for (int i = 0; i < kEl; ++i) gv[i] = gamma[tid + i * 64 * kQWaves];
+    lds_barrier();
+    float h[NB][NV];  // this lane's activations, for every row it works on
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int i = 0; i < kEl; ++i) xv[b][i] = b < B ? x[(size_t)b * x_stride + tid + i * 64 * kQWaves] : 0.f;
-    // Q4_K blocks (144 bytes) are whole 16-byte pieces: each lane loads the two pieces each of its
-    // items needs (the block's header with d, dmin and the scales; the item's 16 bytes of nibbles) and
-    // decodes from registers, without staging the row through LDS (5.73-5.75 against 6.07-6.08 us at
-    // Qwen3-4B).  Q8_0 (34-byte) and Q6_K (210-byte) blocks are not piece-aligned and stay staged.
-    constexpr bool kDirect = T == 12;
-    u32x4_t dh[kDirect ? E / 512 : 1], dq[kDirect ? E / 512 : 1];
-    if constexpr (kDirect) {
+        for (int k = 0; k < NV; k += 4) {
+            const float4 v = *reinterpret_cast<const float4*>(
+                hs + b * S::kHRow + S::h_at(S::first(k / S::kPer, li) + k % S::kPer));
+            h[b][k] = v.x, h[b][k + 1] = v.y, h[b][k + 2] = v.z, h[b][k + 3] = v.w;
+        }
+
+    // ---- the rows, RB at a time.  Every batch but the last loads each row's registers again as soon as
+    // they are used, unconditionally (a branch around a load would make the waits behind it count the
+    // worst case, that is, wait for everything)
+    const int turns = (row_hi - row_lo + S::kGroups - 1) / S::kGroups;
+    auto batch = [&](int j0, int buf, auto more) {
+        float acc[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) acc[k] = 0.f;
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            if (more || j0 + i < turns) {
+                float wf[NV];
+                wt[i].values(li, wf);
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    float a = wf[0] * h[b][0];
+#pragma unroll
+                    for (int k = 1; k < NV; ++k) a = fmaf(wf[k], h[b][k], a);
+                    acc[i * NB + b] = a;
+                }
+            }
+            if constexpr (more) wt[i].load(w + (size_t)row_at(j0 + RB + i) * W::kRowBytes, li);
+            __builtin_amdgcn_sched_barrier(0);  // one row's values in registers at a time
+        }
+        int at = 0, n = N;
+        half_wave_sums<16, N>(acc, lane, at, n);
+#pragma unroll
+        for (int k = 0; k < (N + 31) / 32; ++k)
+            if (k < n) red[buf][hwave][at + k] = acc[k];
+        lds_barrier();  // (two buffers: the next batch's stores meet no reader of this one)
+        for (int t = tid; t < S::kGroups * N; t += S::kThreads) {
+            const int g = t / N, v = t - g * N, i = v / NB, b = v - i * NB;
+            const int row = row_lo + g + (j0 + i) * S::kGroups;
+            float sum = 0.f;
+#pragma unroll
+            for (int k = 0; k < HW; ++k) sum += red[buf][g * HW + k][v];
+            if (row < row_hi) out[(size_t)b * out_stride + row] = sum;
+        }
+    };
+    int j0 = 0, buf = 0;
+    for (; j0 + RB < turns; j0 += RB, buf ^= 1) batch(j0, buf, std::true_type{});
+    batch(j0, buf, std::false_type{});
+}
+
+// ------------------------------------------------------------------ one activation row, a wave to two rows
+// With a single activation row the sums need no sharing, and at the hidden sizes whose rows take ten waves
+// above (160 or 320 lanes: 2560 and 5120) a wave per two output rows with every byte of them in flight is
+// the faster layout: four waves to a workgroup, the normed activations read from LDS, no reduction beyond the
+// wave (as it is for F32 at 2048, whose 16 rows a CU are too few to keep rows in flight behind others).  Graph-timed, this against the kernel above: F32 11.35 / 11.63 us at E 2560 and 24.7 / 25.6 at 5120, F16
+// 7.31 / 7.23 and 14.5 / 15.3, Q8_0 7.03 / 7.89 and 14.1 / 14.7, Q4_K 5.86 / 6.40 and 11.0 / 11.4 (Q6_K 8.36 /
+// 8.09 and 18.7 / 15.8: taken above), F32 7.34 / 7.82 at E 2048.
+constexpr int kOneWaves = 4, kOneRows = 2;  // waves per workgroup, rows per wave
+
+template <int T, int E>
+constexpr bool project_one_row() {
+    return (T != 14 && (E == 2560 || E == 5120)) || (T == 0 && E == 2048);
+}
+
+// RMSNorm of the activation row into hs (src/ops.cpp:155-160), kEl elements per thread; the caller's barrier
+// makes it visible.
+template <int E, int kEl>
+__device__ __forceinline__ void norm_one(const float (&xv)[kEl], const float (&gv)[kEl], float eps, float* hs,
+                                         double* ssum) {
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    double ss = 0.0;
+#pragma unroll
+    for (int i = 0; i < kEl; ++i) ss += (double)xv[i] * (double)xv[i];
+    ss = wave_sum_f64(ss);
+    if (lane == 0) ssum[wv] = ss;
+    __syncthreads();
+    ss = 0.0;
+#pragma unroll
+    for (int k = 0; k < kOneWaves; ++k) ss += ssum[k];
+    const float inv = (float)(1.0 / sqrt(ss / (double)E + (double)eps));
+#pragma unroll
+    for (int i = 0; i < kEl; ++i) {
+#pragma clang fp contract(off)
+        hs[tid + i * 64 * kOneWaves] = (xv[i] * inv) * gv[i];
+    }
+}
+
+// F32 and F16: lane l reads 16-byte pieces l, l + 64, ... of both rows.
+template <int T, int E>
+__global__ __launch_bounds__(64 * kOneWaves) void k_qkv_project_one(const float* __restrict__ x,
+                                                                    const float* __restrict__ gamma, float eps,
+                                                                    const uint8_t* __restrict__ w, int n_out,
+                                                                    float* __restrict__ out) {
+    constexpr int kPer = T == 1 ? 8 : 4, P = E / kPer / 64, kEl = E / (64 * kOneWaves);
+    __shared__ __align__(16) float hs[E];
+    __shared__ double ssum[kOneWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int r0 = (blockIdx.x * kOneWaves + wv) * kOneRows;
+    // the activation and gamma elements first, then every weight piece of the wave's rows: loads return in
+    // order, so the norm waits for the activations only and overlaps the weight stream
+    float xv[kEl], gv[kEl];
+#pragma unroll
+    for (int i = 0; i < kEl; ++i) gv[i] = gamma[tid + i * 64 * kOneWaves];
+#pragma unroll
+    for (int i = 0; i < kEl; ++i) xv[i] = x[tid + i * 64 * kOneWaves];
+    u32x4_t wr[kOneRows][P];
+#pragma unroll
+    for (int rr = 0; rr < kOneRows; ++rr) {
+        const uint8_t* row = w + (size_t)min(r0 + rr, n_out - 1) * E * (T == 1 ? 2 : 4);
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+            wr[rr][p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(row) + p * 64 + lane);
+    }
+    norm_one<E>(xv, gv, eps, hs, ssum);
+    __syncthreads();
+    float acc[kOneRows] = {};
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int e0 = (p * 64 + lane) * kPer;
+#pragma unroll
+        for (int rr = 0; rr < kOneRows; ++rr) {
+            float wf[kPer];
+            if constexpr (T == 1) {
+                f16x8(wr[rr][p], wf);
+            } else {
+                wf[0] = __uint_as_float(wr[rr][p].x), wf[1] = __uint_as_float(wr[rr][p].y);
+                wf[2] = __uint_as_float(wr[rr][p].z), wf[3] = __uint_as_float(wr[rr][p].w);
+            }
+#pragma unroll
+            for (int k = 0; k < kPer; k += 4) {
+                const float4 h4 = *reinterpret_cast<const float4*>(hs + e0 + k);
+                acc[rr] = fmaf(wf[k], h4.x, acc[rr]);
+                acc[rr] = fmaf(wf[k + 1], h4.y, acc[rr]);
+                acc[rr] = fmaf(wf[k + 2], h4.z, acc[rr]);
+                acc[rr] = fmaf(wf[k + 3], h4.w, acc[rr]);
+            }
+        }
+    }
+#pragma unroll
+    for (int rr = 0; rr < kOneRows; ++rr) {
+        const float s = wave_sum(acc[rr]);
+        if (lane == 0 && r0 + rr < n_out) out[r0 + rr] = s;
+    }
+}
+
+// Q4_K and Q8_0: lanes of even and odd index take the two rows, lane l items l / 2, l / 2 + 32, ....  Q4_K
+// items are whole 16-byte pieces and load straight into registers; Q8_0 rows (34-byte blocks) come in as
+// coalesced pieces and are parked in a wave-private LDS area first.
+template <int T, int E>
+__global__ __launch_bounds__(64 * kOneWaves) void k_qkv_project_one_q(const float* __restrict__ x,
+                                                                      const float* __restrict__ gamma, float eps,
+                                                                      const uint8_t* __restrict__ w, int n_out,
+                                                                      float* __restrict__ out) {
+    using W = Weights<T, E>;
+    constexpr int RB = (int)W::kRowBytes, kEl = E / (64 * kOneWaves), kItems = E / 512;
+    constexpr int kPieces = (RB / 16 + 63) / 64;  // staged: 16-byte pieces per lane per row
+    constexpr bool kStaged = T == 8;
+    static_assert(RB % 16 == 0 && E % 512 == 0, "hidden size");
+    __shared__ __align__(16) float hs[E];
+    __shared__ __align__(16) uint8_t rows[kStaged ? kOneWaves * kOneRows * RB : 16];
+    __shared__ double ssum[kOneWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int r0 = (blockIdx.x * kOneWaves + wv) * kOneRows;
+    float xv[kEl], gv[kEl];
+#pragma unroll
+    for (int i = 0; i < kEl; ++i) gv[i] = gamma[tid + i * 64 * kOneWaves];
+#pragma unroll
+    for (int i = 0; i < kEl; ++i) xv[i] = x[tid + i * 64 * kOneWaves];
+    W it[kStaged ? 1 : kItems];
+    u32x4_t pc[kOneRows][kStaged ? kPieces : 1];
+    if constexpr (kStaged) {
+#pragma unroll
+        for (int rr = 0; rr < kOneRows; ++rr) {
+            const uint8_t* row = w + (size_t)min(r0 + rr, n_out - 1) * RB;
+#pragma unroll
+            for (int k = 0; k < kPieces; ++k)  // clamped: the tail lanes reload the last piece
+                pc[rr][k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(row) +
+                                                       min(lane + 64 * k, RB / 16 - 1));
+        }
+    } else {
         const uint8_t* row = w + (size_t)min(r0 + (lane & 1), n_out - 1) * RB;
 #pragma unroll
-        for (int j = 0; j < E / 512; ++j) {
-            const int k = (lane >> 1) + 32 * j, v = (k & 15) * 16;
-            const uint8_t* blk = row + 144 * (k >> 4);
-            dh[j] = *reinterpret_cast<const u32x4_t*>(blk);
-            dq[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(blk + 16 + 32 * (v >> 6) + (v & 31)));
-        }
+        for (int j = 0; j < kItems; ++j) it[j].load(row, (lane >> 1) + 32 * j);
     }
-    u32x4_t pc[kQRowsPerWave][wide ? kPer : 1];
-    uint32_t pd[kQRowsPerWave][wide ? 1 : kPer];
+    norm_one<E>(xv, gv, eps, hs, ssum);
+    uint8_t* my_rows = rows + wv * kOneRows * RB;
+    if constexpr (kStaged) {
 #pragma unroll
-    for (int rr = 0; rr < kQRowsPerWave; ++rr) {
-        if (kDirect) break;
-        const uint8_t* row = w + (size_t)min(r0 + rr, n_out - 1) * RB;
+        for (int rr = 0; rr < kOneRows; ++rr)
 #pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const int p = min(lane + 64 * k, RB / kPiece - 1);  // clamped: the tail lanes reload the last piece
-            if constexpr (wide) pc[rr][k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(row) + p);
-            else pd[rr][k] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(row) + p);
-        }
-    }
-
-    // ---- attention RMSNorm of the B rows into LDS (src/ops.cpp:155-160), as the float kernels
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        double ss = 0.0;
-#pragma unroll
-        for (int i = 0; i < kEl; ++i) ss += (double)xv[b][i] * (double)xv[b][i];
-        ss = wave_sum_f64(ss);
-        if (lane == 0) ssum[wv][b] = ss;
+            for (int k = 0; k < kPieces; ++k)
+                if (lane + 64 * k < RB / 16) reinterpret_cast<u32x4_t*>(my_rows + rr * RB)[lane + 64 * k] = pc[rr][k];
     }
     __syncthreads();
+    float acc = 0.f;
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        if (b >= B) break;
-        double ss = 0.0;
-#pragma unroll
-        for (int k = 0; k < kQWaves; ++k) ss += ssum[k][b];
-        const float inv = (float)(1.0 / sqrt(ss / (double)E + (double)eps));
-#pragma unroll
-        for (int i = 0; i < kEl; ++i) {
-#pragma clang fp contract(off)
-            hs[b * E + tid + i * 64 * kQWaves] = (xv[b][i] * inv) * gv[i];
-        }
-    }
-
-    // ---- the row bytes into this wave's LDS area (sized for B activation rows)
-    uint8_t* qrow = reinterpret_cast<uint8_t*>(hs + B * E) + (size_t)wv * kQRowsPerWave * RB;
-#pragma unroll
-    for (int rr = 0; rr < kQRowsPerWave; ++rr) {
-        if (kDirect) break;
-        uint8_t* dst = qrow + rr * RB;
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const int p = lane + 64 * k;
-            if (p < RB / kPiece) {
-                if constexpr (wide) reinterpret_cast<u32x4_t*>(dst)[p] = pc[rr][k];
-                else reinterpret_cast<uint32_t*>(dst)[p] = pd[rr][k];
-            }
-        }
-    }
-    __syncthreads();  // the activations of every wave and this wave's row bytes
-
-    // ---- decode items of 16 values and accumulate: lane l works on row l & 1, items l / 2,
-    // l / 2 + 32, ... of it; the lanes of one row are summed at the end
-    const int rr = lane & 1;
-    const uint8_t* myrow = qrow + rr * RB;
-    float acc[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) acc[b] = 0.f;
-#pragma unroll
-    for (int j = 0; j < E / 512; ++j) {
+    for (int j = 0; j < kItems; ++j) {
         const int k = (lane >> 1) + 32 * j;
         float wf[16];
-        if constexpr (kDirect) {
-            const int v = (k & 15) * 16;
-            decode16_q4k_regs(dh[j], dq[j], 2 * (v >> 6) + ((v >> 5) & 1), (v >> 5) & 1, wf);
+        if constexpr (kStaged) {
+            const uint8_t* blk = my_rows + (lane & 1) * RB + 34 * (k >> 1);
+            __builtin_memcpy(&it[0].q, blk + 2 + 16 * (k & 1), 16);  // 2-byte aligned
+            it[0].d16 = *reinterpret_cast<const uint16_t*>(blk);
+            it[0].values(k, wf);
         } else {
-            decode16<T>(myrow, k, wf);
+            it[j].values(k, wf);
         }
+        // an item's activations are read once the sum before it is known: all items' at once would take the
+        // registers of two waves a SIMD (Q4_K, E 5120: 12.4 against 11.1 us)
+        int at = 16 * k;
+        asm volatile("" : "+v"(at), "+v"(acc));
+        const float4* hp = reinterpret_cast<const float4*>(hs + at);
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            if (b >= B) break;
-            const float4* hp = reinterpret_cast<const float4*>(hs + b * E + 16 * k);
-            float a = acc[b];
-#pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-                const float4 hv = hp[q4];
-                a = fmaf(wf[4 * q4], hv.x, a);
-                a = fmaf(wf[4 * q4 + 1], hv.y, a);
-                a = fmaf(wf[4 * q4 + 2], hv.z, a);
-                a = fmaf(wf[4 * q4 + 3], hv.w, a);
-            }
-            acc[b] = a;
+        for (int q4 = 0; q4 < 4; ++q4) {
+            const float4 hv = hp[q4];
+            acc = fmaf(wf[4 * q4], hv.x, acc);
+            acc = fmaf(wf[4 * q4 + 1], hv.y, acc);
+            acc = fmaf(wf[4 * q4 + 2], hv.z, acc);
+            acc = fmaf(wf[4 * q4 + 3], hv.w, acc);
         }
     }
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        if (b >= B) break;
-        float sres = acc[b];  // sum over the 32 lanes of this lane's row (xor 2 .. 32 keep the parity)
-        sres += lane_xor<2>(sres);
-        sres += lane_xor<4>(sres);
-        sres += lane_xor<8>(sres);
-        sres += lane_xor<16>(sres);
-        sres += lane_xor<32>(sres);
-        if (lane < 2 && r0 + rr < n_out) out[(size_t)b * out_stride + r0 + rr] = sres;
-    }
-}
-
-static size_t qkv_project_q_lds(int E, int w_type, int B) {
-    const int vals = w_type == 8 ? 32 : 256, bytes = w_type == 8 ? 34 : w_type == 12 ? 144 : 210;
-    const size_t rb = (size_t)(E / vals) * bytes;
-    return (size_t)B * E * sizeof(float) + (size_t)kQWaves * kQRowsPerWave * rb;
-}
-
-template <int T, int NB, int E>
-static hipError_t launch_q_nbe(hipStream_t st, const float* x, long x_stride, int B, const float* gamma, float eps,
-                               const void* w, int n_out, float* out, long out_stride) {
-    static std::atomic<bool> opted;
-    if (const hipError_t e = opt_in_lds(opted, (const void*)k_qkv_project_q<T, NB, E>, 150 * 1024); e != hipSuccess)
-        return e;
-    const int per_block = kQWaves * kQRowsPerWave;
-    k_qkv_project_q<T, NB, E><<<(n_out + per_block - 1) / per_block, 64 * kQWaves, qkv_project_q_lds(E, T, B), st>>>(
-        x, x_stride, B, gamma, eps, static_cast<const uint8_t*>(w), n_out, out, out_stride);
-    return hipGetLastError();
-}
-
-template <int T, int NB>
-static hipError_t launch_q_nb(hipStream_t st, const float* x, long x_stride, int B, int E, const float* gamma,
-                              float eps, const void* w, int n_out, float* out, long out_stride) {
-#define EI_PROJ_QE(EE) \
-    case EE: return launch_q_nbe<T, NB, EE>(st, x, x_stride, B, gamma, eps, w, n_out, out, out_stride);
-    switch (E) {
-        EI_PROJ_QE(1024) EI_PROJ_QE(2048) EI_PROJ_QE(2560) EI_PROJ_QE(4096) EI_PROJ_QE(5120)
-        default: return hipErrorInvalidValue;
-    }
-#undef EI_PROJ_QE
-}
-
-template <int T>
-static hipError_t launch_q(hipStream_t st, const float* x, long x_stride, int B, int E, const float* gamma, float eps,
-                           const void* w, int n_out, float* out, long out_stride) {
-    if (B <= 1) return launch_q_nb<T, 1>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
-    if (B <= 2) return launch_q_nb<T, 2>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
-    return launch_q_nb<T, 4>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
+    acc += lane_xor<2>(acc);  // sum over the 32 lanes of this lane's row (xor 2 .. 32 keep the parity)
+    acc += lane_xor<4>(acc);
+    acc += lane_xor<8>(acc);
+    acc += lane_xor<16>(acc);
+    acc += lane_xor<32>(acc);
+    if (lane < 2 && r0 + lane < n_out) out[r0 + lane] = acc;
 }
 
 int qkv_project_max_rows(int E) {
@@ -495,55 +580,95 @@ bool qkv_project_built(int E, int w_type) {
     return E == 1024 || E == 2048 || E == 2560 || E == 4096 || E == 5120;
 }
 
-template <bool WF16, int NB, int P>
-static hipError_t launch_nbp(hipStream_t st, const float* x, long x_stride, int B, int E, const float* gamma,
-                             float eps, const void* w, int n_out, float* out, long out_stride) {
-    const size_t lds = (size_t)B * E * sizeof(float);
-    static std::atomic<bool> opted;
-    if (const hipError_t e = opt_in_lds(opted, (const void*)k_qkv_project<WF16, NB, P>, kProjMaxLdsFloats * 4);
-        e != hipSuccess)
-        return e;
-    const int per_block = kProjWaves * kRowsPerWave;
-    k_qkv_project<WF16, NB, P><<<(n_out + per_block - 1) / per_block, 64 * kProjWaves, lds, st>>>(
-        x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
-    return hipGetLastError();
-}
-
-template <bool WF16, int NB>
-static hipError_t launch_nb(hipStream_t st, const float* x, long x_stride, int B, int E, const float* gamma, float eps,
-                            const void* w, int n_out, float* out, long out_stride) {
-#define EI_PROJ_P(PP) \
-    case PP: return launch_nbp<WF16, NB, PP>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
-    if constexpr (WF16) {
-        switch (qkv_project_pieces(E, true)) {
-            EI_PROJ_P(2) EI_PROJ_P(4) EI_PROJ_P(5) EI_PROJ_P(8) EI_PROJ_P(10) EI_PROJ_P(16) EI_PROJ_P(20)
-            default: return hipErrorInvalidValue;
-        }
+template <int T, int NB, int E>
+static hipError_t launch_t(hipStream_t st, const float* x, long x_stride, const float* gamma, float eps,
+                           const void* w, int n_out, float* out, long out_stride) {
+    if constexpr (NB == 1 && project_one_row<T, E>()) {
+        constexpr int kPerWg = kOneWaves * kOneRows;
+        const dim3 grid((n_out + kPerWg - 1) / kPerWg);
+        if constexpr (T <= 1)
+            k_qkv_project_one<T, E><<<grid, 64 * kOneWaves, 0, st>>>(x, gamma, eps, static_cast<const uint8_t*>(w),
+                                                                     n_out, out);
+        else
+            k_qkv_project_one_q<T, E><<<grid, 64 * kOneWaves, 0, st>>>(x, gamma, eps, static_cast<const uint8_t*>(w),
+                                                                       n_out, out);
+        return hipGetLastError();
     } else {
-        switch (qkv_project_pieces(E, false)) {
-            EI_PROJ_P(4) EI_PROJ_P(8) EI_PROJ_P(10) EI_PROJ_P(16) EI_PROJ_P(20)
-            default: return hipErrorInvalidValue;
+        using S = RowShape<T, E>;
+        // one workgroup a CU
+        const int rows = (n_out + 255) / 256, turns = (rows + S::kGroups - 1) / S::kGroups;
+        // rows in flight: as many as the registers (256 or 168 a lane at 8 or 10 waves) take beside the
+        // activations and one row's values, at most 8; fewer where the workgroup's rows then come out in even
+        // batches
+        constexpr int kRegs = sizeof(Weights<T, E>) / 4;
+        constexpr int kBudget = S::kThreads <= 512 ? 160 : 112;
+        constexpr int kFit = (kBudget - S::kVals * NB) / (kRegs + NB);
+        constexpr int kMost = kFit >= 8 ? 8 : kFit >= 6 ? 6 : kFit >= 4 ? 4 : kFit >= 3 ? 3 : 2;
+        const int batches = (turns + kMost - 1) / kMost, want = (turns + batches - 1) / batches;
+        constexpr size_t lds = (size_t)NB * S::kHRow * sizeof(float);
+        auto go = [&](auto rb) {
+            static std::atomic<bool> opted;
+            if (const hipError_t e = opt_in_lds(opted, (const void*)k_qkv_project<T, NB, E, rb>, lds); e != hipSuccess)
+                return e;
+            k_qkv_project<T, NB, E, rb><<<(n_out + rows - 1) / rows, S::kThreads, lds, st>>>(
+                x, x_stride, gamma, eps, static_cast<const uint8_t*>(w), n_out, rows, out, out_stride);
+            return hipGetLastError();
+        };
+        if constexpr (kMost > 2) {
+            if (want <= 2) return go(std::integral_constant<int, 2>{});
         }
+        if constexpr (kMost > 3 && T > 1) {
+            if (want <= 3) return go(std::integral_constant<int, 3>{});
+        }
+        if constexpr (kMost > 4) {
+            if (want <= 4) return go(std::integral_constant<int, 4>{});
+        }
+        if constexpr (kMost > 6) {
+            if (want <= 6) return go(std::integral_constant<int, 6>{});
+        }
+        return go(std::integral_constant<int, kMost>{});
     }
-#undef EI_PROJ_P
 }
 
-template <bool WF16>
+template <int T, int NB>
+static hipError_t launch_e(hipStream_t st, const float* x, long x_stride, int E, const float* gamma, float eps,
+                           const void* w, int n_out, float* out, long out_stride) {
+#define EI_PROJ_E(EE) \
+    case EE: return launch_t<T, NB, EE>(st, x, x_stride, gamma, eps, w, n_out, out, out_stride);
+    switch (E) {
+        EI_PROJ_E(1024) EI_PROJ_E(2048) EI_PROJ_E(2560) EI_PROJ_E(4096) EI_PROJ_E(5120)
+        default: break;
+    }
+    if constexpr (T == 1 && NB * 8192 <= kProjMaxLdsFloats) {
+        if (E == 8192) return launch_t<T, NB, 8192>(st, x, x_stride, gamma, eps, w, n_out, out, out_stride);
+    }
+    if constexpr (T == 1 && NB * 10240 <= kProjMaxLdsFloats) {
+        if (E == 10240) return launch_t<T, NB, 10240>(st, x, x_stride, gamma, eps, w, n_out, out, out_stride);
+    }
+#undef EI_PROJ_E
+    return hipErrorInvalidValue;
+}
+
+template <int T>
 static hipError_t launch_w(hipStream_t st, const float* x, long x_stride, int B, int E, const float* gamma, float eps,
                            const void* w, int n_out, float* out, long out_stride) {
-    if (B <= 1) return launch_nb<WF16, 1>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
-    if (B <= 2) return launch_nb<WF16, 2>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
-    return launch_nb<WF16, 4>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
+    switch (B) {
+        case 1: return launch_e<T, 1>(st, x, x_stride, E, gamma, eps, w, n_out, out, out_stride);
+        case 2: return launch_e<T, 2>(st, x, x_stride, E, gamma, eps, w, n_out, out, out_stride);
+        case 3: return launch_e<T, 3>(st, x, x_stride, E, gamma, eps, w, n_out, out, out_stride);
+        case 4: return launch_e<T, 4>(st, x, x_stride, E, gamma, eps, w, n_out, out, out_stride);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 hipError_t launch_qkv_project(hipStream_t st, const float* x, long x_stride, int B, int E, const float* gamma,
                               float eps, const void* w, int w_type, int n_out, float* out, long out_stride) {
     switch (w_type) {
-        case 0: return launch_w<false>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
-        case 1: return launch_w<true>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
-        case 8: return launch_q<8>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
-        case 12: return launch_q<12>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
-        case 14: return launch_q<14>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
+        case 0: return launch_w<0>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
+        case 1: return launch_w<1>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
+        case 8: return launch_w<8>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
+        case 12: return launch_w<12>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
+        case 14: return launch_w<14>(st, x, x_stride, B, E, gamma, eps, w, n_out, out, out_stride);
         default: return hipErrorInvalidValue;
     }
 }
