@@ -9,6 +9,7 @@ The names follow the reference's per-layer attention steps (src/cuda/model_cuda.
 """
 from __future__ import annotations
 
+import functools
 from dataclasses import dataclass
 
 import torch
@@ -19,7 +20,9 @@ HEAD_DIM = 128
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the raw handle of torch's current stream: torch.cuda.current_stream() builds a Stream object around it
+    # (2.6 us against 0.25 us, every call; a decode step's two launches take 7.2 us)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -35,8 +38,10 @@ def _need_gpu_f32(name: str, t: torch.Tensor) -> None:
         raise ValueError(f"{name} must be contiguous in its last dimension")
 
 
+@functools.lru_cache(maxsize=None)
 def default_scale(head_dim: int = HEAD_DIM) -> float:
-    """1/sqrt(D) rounded to float as the reference does (src/model.cpp:163, src/cuda/model_cuda.cu:1786)."""
+    """1/sqrt(D) rounded to float as the reference does (src/model.cpp:163, src/cuda/model_cuda.cu:1786).
+    A number per head_dim, so it is computed once (4.1 us of tensor operations in every call before)."""
     return float(torch.tensor(1.0, dtype=torch.float32) / torch.sqrt(torch.tensor(float(head_dim),
                                                                                   dtype=torch.float32)))
 
