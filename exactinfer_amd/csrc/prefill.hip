@@ -90,7 +90,7 @@ constexpr int kKS = 2;                           // key groups per workgroup
 constexpr float kLazy = 8.f;                     // lazy-rescale threshold (log2 units)
 constexpr int kXchF = 34;                        // floats per lane exchanged by the merge
 constexpr int kSlots = 4;                        // query slots (waves) per key group
-constexpr int kPassTiles = 3;                    // a pass's fixed cost, in tiles (key-share balance; 1..4 tried)
+constexpr int kPassTiles = 5;                    // a pass's fixed cost, in tiles (key-share balance)
 
 // n / d for small d (1..8) and n * d < 2^32 as one multiply-high: the per-pass index math
 // runs on the scalar unit, which the eight waves of a CU share, so a division loop per use
@@ -106,7 +106,8 @@ __device__ __forceinline__ int fdiv(int n, FastDiv f) {
 // shares, the pair's tiles, unit pair's then unit nu-1-pair's, are cut into ksplit contiguous
 // shares of equal cost, where the boundary between the units counts as kPassTiles extra tiles:
 // a share that crosses it runs two passes (q staging, first tiles, key-group merge and store
-// twice), so it gets that many fewer tiles, and every other share runs one pass.  Share
+// twice), so it gets that many fewer tiles, and every other share runs one pass (3 to 8 tried, 512
+// tokens at 0 / 1536, G = 4: 47.2 / 96.0 us at 3, 45.8 / 94.0 at 4 and 5, 47.5 / 93.9 at 6, 49.3 / 95.0 at 8).  Share
 // `split` holds tiles [lo0, lo0 + r0) of unit pair and [lo1, lo1 + r1) of unit nu-1-pair; a
 // unit without tiles in a share has no pass there and no partial, and k_prefill_combine,
 // which evaluates the same cut, does not read one.  With ksplit = 1 the share is both units.
