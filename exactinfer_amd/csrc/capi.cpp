@@ -448,11 +448,31 @@ EI_API size_t ei_attn_prefill_ws_bytes(int max_B, int n_head, int n_head_kv, int
     if (n_head_kv > kMaxKvHeads || !prefill_rows_ok(max_B, n_head)) return 0;
     size_t most = 0;  // the plan varies with B: size for every chunk of up to max_B rows
     for (int b = 1; b <= max_B; ++b) {
-        const size_t need = ei::prefill_ws_bytes(b, n_head, n_head_kv, max_kv);
+        // (the fine plan never has fewer shares than the other)
+        const size_t need = ei::prefill_ws_bytes(b, n_head, ei::prefill_split(b, n_head, n_head_kv, max_kv, true));
         if (need > most) most = need;
     }
     return most;
 }
+
+namespace {
+
+// Key shares of a chunk: the plan whose shares hold at least four tiles (`coarse`), whose workspace every
+// call has to bring, or the fine one where the workspace holds that.
+struct PrefillPlan {
+    int coarse, ksplit;
+};
+int prefill_plan(int B, int n_head, int n_head_kv, int max_kv, const void* ws, size_t ws_bytes, PrefillPlan* p) {
+    p->coarse = p->ksplit = ei::prefill_split(B, n_head, n_head_kv, max_kv, false);
+    const size_t need = ei::prefill_ws_bytes(B, n_head, p->coarse);
+    REQUIRE(ws_bytes >= need, "workspace %zu B < %zu B (ei_attn_prefill_ws_bytes)", ws_bytes, need);
+    REQUIRE(need == 0 || (ws && aligned16(ws)), "workspace must be a 16-byte aligned device pointer");
+    const int fine = ei::prefill_split(B, n_head, n_head_kv, max_kv, true);
+    if (ws && aligned16(ws) && ws_bytes >= ei::prefill_ws_bytes(B, n_head, fine)) p->ksplit = fine;
+    return EI_OK;
+}
+
+}  // namespace
 
 EI_API int ei_attn_prefill_split(ei_stream_t stream, const float* q, long q_stride, float* out, const float* kc,
                                  const float* vc, const int* pos_dev, int B, int n_head, int n_head_kv, int head_dim,
@@ -466,12 +486,10 @@ EI_API int ei_attn_prefill_split(ei_stream_t stream, const float* q, long q_stri
     REQUIRE(q_stride >= (long)n_head * head_dim && q_stride % 4 == 0, "q_stride %ld", q_stride);
     REQUIRE(aligned16(q) && aligned16(out) && aligned16(kc) && aligned16(vc), "pointers must be 16-byte aligned");
     if (B == 0) return ok();
-    const int ksplit = ei::prefill_split(B, n_head, n_head_kv, max_kv);
-    const size_t need = ei::prefill_ws_bytes(B, n_head, n_head_kv, max_kv);
-    REQUIRE(ws_bytes >= need, "workspace %zu B < %zu B (ei_attn_prefill_ws_bytes)", ws_bytes, need);
-    REQUIRE(need == 0 || (ws && aligned16(ws)), "workspace must be a 16-byte aligned device pointer");
+    PrefillPlan plan;
+    if (int e = prefill_plan(B, n_head, n_head_kv, max_kv, ws, ws_bytes, &plan)) return e;
     return hip_status(ei::launch_prefill(static_cast<hipStream_t>(stream), q, q_stride, out, kc, vc, pos_dev, B,
-                                         n_head, n_head_kv, scale, ksplit, ws),
+                                         n_head, n_head_kv, scale, plan.ksplit, ws),
                       "prefill launch");
 }
 
@@ -493,26 +511,23 @@ int prefill_step_impl(ei_stream_t stream, float* qkv, long row_stride, float* ou
     REQUIRE(aligned16(qkv) && aligned16(out) && aligned16(kc) && aligned16(vc) && row_stride % 4 == 0,
             "pointers and row_stride must be 16-byte aligned");
     if (B == 0) return ok();
-    const int ksplit = ei::prefill_split(B, n_head, n_head_kv, max_kv);
-    const size_t need = ei::prefill_ws_bytes(B, n_head, n_head_kv, max_kv);
-    REQUIRE(ws_bytes >= need, "workspace %zu B < %zu B (ei_attn_prefill_ws_bytes)", ws_bytes, need);
-    REQUIRE(need == 0 || (ws && aligned16(ws)), "workspace must be a 16-byte aligned device pointer");
+    PrefillPlan plan;
+    if (int e = prefill_plan(B, n_head, n_head_kv, max_kv, ws, ws_bytes, &plan)) return e;
     const hipStream_t st = static_cast<hipStream_t>(stream);
     // the attention kernel norms q itself (full-width RoPE, every Qwen3) when the key range is
-    // split over at most four shares: each share norms the q rows of the units it runs (one
-    // pass for most shares), which costs less than the q traffic it saves in the prologue
-    // (512-token chunks, 4 shares: chunk step 90.7 -> 91.3 TFLOP/s); with more shares the
-    // prologue norms every head in place first (the paged variant always takes the full
+    // split over at most four shares (of at least four tiles): each share norms the q rows of the
+    // units it runs, and q stays as it is in qkv; with more shares the prologue norms every head in place first (the paged variant always takes the full
     // prologue: the in-kernel norm and the block table together exceed the attention kernel's
     // register budget)
-    const bool fuse_q = rope_dim == head_dim && ksplit <= 4 && block_table == nullptr;
+    const bool fuse_q = rope_dim == head_dim && plan.coarse <= 4 && block_table == nullptr;
     if (int e = hip_status(ei::launch_qkv_prepare(st, qkv, B, row_stride, n_head, n_head_kv, q_gamma, k_gamma, cs,
                                                   pos_dev, rope_dim, eps, kc, vc, fuse_q ? n_head : 0, block_table,
                                                   block_shift, max_blocks),
                            "prefill step: prologue launch"))
         return e;
-    return hip_status(ei::launch_prefill(st, qkv, row_stride, out, kc, vc, pos_dev, B, n_head, n_head_kv, scale, ksplit,
-                                         ws, fuse_q ? q_gamma : nullptr, cs, eps, block_table, block_shift, max_blocks),
+    return hip_status(ei::launch_prefill(st, qkv, row_stride, out, kc, vc, pos_dev, B, n_head, n_head_kv, scale,
+                                         plan.ksplit, ws, fuse_q ? q_gamma : nullptr, cs, eps, block_table, block_shift,
+                                         max_blocks),
                       "prefill step: attention launch");
 }
 

@@ -131,8 +131,9 @@ hipError_t launch_qkv_project(hipStream_t st, const float* x, long x_stride, int
 // Key split across workgroups for short chunks: ksplit shares per query block, merged by a
 // second launch; fixed by (B, max_kv) so graphs replay unchanged.
 constexpr int kPrefillMaxSplit = 8;
-int prefill_split(int B, int H, int HKV, int max_kv);
-size_t prefill_ws_bytes(int B, int H, int HKV, int max_kv);  // 0 when no split is planned
+// fine: shares of as little as one tile (a larger workspace)
+int prefill_split(int B, int H, int HKV, int max_kv, bool fine);
+size_t prefill_ws_bytes(int B, int H, int ksplit);  // 0 for one share
 // q_gamma != nullptr: the q rows are raw projections; the kernel applies QK-norm + full-width
 // RoPE (table cs of rope_dim 128, eps) to each row where it stages it, leaving the q buffer
 // untouched.  block_table != nullptr: the keys sit in a paged pool (block size 2^block_shift >= 32;

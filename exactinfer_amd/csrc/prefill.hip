@@ -751,17 +751,22 @@ static int prefill_grid1(int B, int H, int HKV) {
     return ((nu + 1) / 2) * HKV;
 }
 
-int prefill_split(int B, int H, int HKV, int max_kv) {
+int prefill_split(int B, int H, int HKV, int max_kv, bool fine) {
     // One workgroup per (unit pair, KV head), all with the same work, one per CU at a time
     // (134 KB of LDS): the launch takes ceil(g1 / 256) rounds.  Splitting every unit's key
     // tiles into k contiguous shares makes g1*k workgroups of 1/k the work, so the time goes
     // as ceil(g1*k / 256) / k.  The plan takes the k in 1..8 with the shortest time, a larger
     // k only when it gains >= 10% (each share adds a combine read and write), and keeps >= 4
     // tiles per share on average (max_kv bounds pos0 + B on the host, which does not see the
-    // device-resident position).
+    // device-resident position).  The fine plan goes down to one tile per share: a tile now costs
+    // about what a share does, and a small chunk leaves most CUs idle otherwise (64 rows at 300, G = 4:
+    // 2 shares 40.8 us, 4 shares 32.7, 8 shares 27.1; 100 rows at 600: 5 shares 38.2, 8 shares 31.6; 16 rows at
+    // 100: 1 share 23.1, 4 shares 20.8; 200 rows at 300, G = 8, paged: 3 shares 45.0, 4 shares 42.4).  It needs a
+    // larger workspace, so a call takes it when its workspace holds it and the other plan when not.
     const int g1 = prefill_grid1(B, H, HKV);
     const long avg_tiles = ((long)max_kv - B / 2 + kKT - 1) / kKT;
-    long kmax = avg_tiles / 4 > 1 ? avg_tiles / 4 : 1;
+    const long kmin_tiles = fine ? 1 : 4;
+    long kmax = avg_tiles / kmin_tiles > 1 ? avg_tiles / kmin_tiles : 1;
     if (kmax > kPrefillMaxSplit) kmax = kPrefillMaxSplit;
     auto rounds = [&](long k) { return (double)((g1 * k + 255) / 256) / (double)k; };
     int best = 1;
@@ -776,11 +781,11 @@ int prefill_split(int B, int H, int HKV, int max_kv) {
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-size_t prefill_ws_bytes(int B, int H, int HKV, int max_kv) {
-    const int k = prefill_split(B, H, HKV, max_kv);
-    if (k <= 1) return 0;
+size_t prefill_ws_bytes(int B, int H, int ksplit) {
+    if (ksplit <= 1) return 0;
     const size_t rows = (size_t)B * H;
-    return align256((size_t)k * rows * kHeadDim * sizeof(float)) + align256((size_t)k * rows * 2 * sizeof(float));
+    return align256((size_t)ksplit * rows * kHeadDim * sizeof(float)) +
+           align256((size_t)ksplit * rows * 2 * sizeof(float));
 }
 
 template <bool kNormQ, bool kPaged>

@@ -20,8 +20,8 @@
 // stream runs on under the arithmetic.  The partial sums of RB rows x NB activation rows are added over
 // 32 lanes by one transposing butterfly and over the half-waves of the group through LDS.
 //
-// Measured, graph-timed per launch, before -> now (us; a plain read of the weights takes 6.2 at 31.5 MB, 8.7 at
-// 50 MB): F16 at E 2560, 6144 outputs, 2 rows 12.6 -> 8.3, 4 rows 24.3 -> 9.9; E 4096, 4 rows 39.4 -> 12.1; E 5120,
+// Measured, graph-timed per launch, before -> now (us; a plain read takes 6.2 at 31.5 MB, 11.5 at
+// 67 MB): F16 at E 2560, 6144 outputs, 2 rows 12.6 -> 8.3, 4 rows 24.3 -> 9.9; E 4096, 4 rows 39.4 -> 12.1; E 5120,
 // 7168 outputs, 4 rows 75.3 -> 17.1; F32 there 66.6 -> 26.1; Q8_0 41.3 -> 16.4; Q4_K 40.1 -> 15.5; Q6_K 48.6 ->
 // 17.1; one row of Q6_K at 5120 18.7 -> 15.8; Q4_K at E 1024, 4096 outputs, 4 rows 5.9 -> 4.5.  Several rows cost
 // little more than one now: the stream bounds them, and what is left over it is the launch's start, the norm

@@ -234,7 +234,8 @@ int ei_attn_prefill(ei_stream_t stream, const float* q, long q_stride, float* ou
  * rounds of the CUs (planned from B and max_kv, an upper bound of *pos_dev + B) and merges the
  * shares with a second launch, using `ws`: ei_attn_prefill_ws_bytes(max_B, ...) bytes serve
  * every chunk of up to max_B rows (0 bytes when no split is planned; the call then equals
- * ei_attn_prefill).  Same semantics and arguments as ei_attn_prefill otherwise; no
+ * ei_attn_prefill).  A smaller workspace is taken too if it holds the plan whose shares have at
+ * least four 32-key tiles each (none is needed where that plan does not split).  Same semantics and arguments as ei_attn_prefill otherwise; no
  * counterpart in the reference beyond k_attn_prefill64.  Calls sharing `ws` must not overlap. */
 size_t ei_attn_prefill_ws_bytes(int max_B, int n_head, int n_head_kv, int max_kv);
 int ei_attn_prefill_split(ei_stream_t stream, const float* q, long q_stride, float* out, const float* kc,
@@ -246,7 +247,7 @@ int ei_attn_prefill_split(ei_stream_t stream, const float* q, long q_stride, flo
  * src/cuda/model_cuda.cu:1800-1820 in two launches (plus the key-split merge when planned).
  * qkv rows [Q|K|V] are raw projections: the K heads are normed + roped in place and appended
  * with the V rows to cache rows *pos_dev + b (as ei_qkv_prepare does).  With rope_dim = 128
- * (every Qwen3) and a plan of at most four key shares, the Q heads are left raw in qkv and
+ * (every Qwen3) and at most four key shares of at least four tiles each, the Q heads are left raw in qkv and
  * normed + roped inside the attention kernel where it stages them; otherwise (a partial
  * rope_dim, or a plan of more shares) they are normed in
  * place by the prologue first.  Same workspace and plan as ei_attn_prefill_split;

@@ -93,3 +93,25 @@ def test_prefill_infinite_and_huge_values(orc, gpu, split):
     cols = [c for c in range(D) if c not in (9, 17, 21)]
     _close(got[..., cols], ref[..., cols])
     assert np.max(np.abs(got[..., 9] / ref[..., 9] - 1.0)) <= 1e-5  # one term rules the column: p's own error
+
+
+@pytest.mark.parametrize("H,HKV,B,pos0", [(32, 8, 16, 100), (16, 8, 64, 40), (8, 1, 33, 0), (40, 8, 100, 20), (4, 1, 2, 61)])
+def test_prefill_small_chunk_plans(orc, gpu, H, HKV, B, pos0):
+    """Small chunks whose plan of at least four tiles a share does not split: the queried workspace
+    gives them finer shares (some hold one tile or none), and a call without a workspace is still
+    taken, unsplit.  Both against float64."""
+    from exactinfer_amd import _capi
+    import torch
+    q, k, v = _inputs(orc, B, pos0, H, HKV, 34000 + B)
+    exact = _exact(q, k, v, pos0, H, HKV)
+    n = pos0 + B
+    ws = gpu.PrefillWorkspace(B, H, HKV, n)
+    assert ws.nbytes > 0
+    _close(_run(gpu, q, k, v, pos0, H, HKV, ws), exact)
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (q, k, v)]
+    pos = torch.tensor([pos0], dtype=torch.int32, device="cuda")
+    out = torch.full((B, H, D), float("nan"), dtype=torch.float32, device="cuda")
+    _capi.call("ei_attn_prefill_split", gpu._stream(), dev[0].data_ptr(), H * D, out.data_ptr(), dev[1].data_ptr(),
+               dev[2].data_ptr(), pos.data_ptr(), B, H, HKV, D, gpu.default_scale(), n, None, 0)
+    torch.cuda.synchronize()
+    _close(out.cpu().numpy(), exact)
