@@ -198,7 +198,9 @@ __device__ __forceinline__ void norm_rope_q8(float* row0, float* row1, const flo
 // ------------------------------------------------------------------ three-plane split
 // x = h + m + l with h, m, l in bf16: h = bf16(x), m = bf16(x - h), l = x - h - m, each rounded to
 // nearest.  Both differences are exact (the residual of a 24-bit value rounded to 8 bits has at
-// most 16 significant bits, the second at most 8), so the three planes hold every bit of x.
+// most 16 significant bits, the second at most 8), so the three planes hold every bit of x as long
+// as none of them leaves bf16's range: from kPlaneMin up, where x's last bit is a normal bf16, to
+// bf16's largest value.  What lies outside is noticed and multiplied in fp32.
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -216,6 +218,11 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t& h, uint32
     m = pk_bf16(ra, rb);
     l = pk_bf16(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xFFFF0000u));
 }
+constexpr float kPlaneMin = 0x1p-100f;
+constexpr float kSmallSum = 0x1p-60f;
+// |x| of a nonzero x in an order of its own, zero last: both tests of a value in one comparison
+__device__ __forceinline__ uint32_t magnitude(uint32_t x) { return (x << 1) - 1u; }
+constexpr uint32_t kTinyMagnitude = (__builtin_bit_cast(uint32_t, kPlaneMin) << 1) - 1u;
 struct Planes {  // eight values: one MFMA operand per plane
     u32x4 h, m, l;
 };
@@ -612,15 +619,37 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
 
         // An infinite K or V value (or a finite one past bf16's range) has no planes to multiply:
         // the residual of inf is NaN, and inf times a zero residual is NaN where the fp32 product is
-        // infinite or the key's weight is zero.  Such a tile shows as a sum that is not finite; the
-        // wave then takes its tiles again in fp32, whose outcome stands whatever it is.
+        // infinite or the key's weight is zero.  Such a tile shows as a sum that is not finite.  A V
+        // value below kPlaneMin may have lost bits of its third plane, which shows only in a sum that is
+        // itself small: weights are at most 2^kLazy and a value is off by at most 2^-134, so over 2^20 keys
+        // a sum from kSmallSum up is off by less than 2^-46 of itself.  A small one has the wave look
+        // through its V tiles, because a column of zeros or of few ordinary values gives one too.  In
+        // both cases the wave then takes its tiles again in fp32, whose outcome stands whatever it is.
         {
-            float z = lsum * 0.f;
+            float z = lsum * 0.f, least = INFINITY;
 #pragma unroll
             for (int db = 0; db < 4; ++db)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) z = __builtin_fmaf(o[db][r], 0.f, z);
-            if (__builtin_amdgcn_ballot_w64(z != 0.f)) {
+                for (int r = 0; r < 16; ++r) {
+                    z = __builtin_fmaf(o[db][r], 0.f, z);
+                    least = fminf(least, __builtin_fabsf(o[db][r]));
+                }
+            uint64_t redo = __builtin_amdgcn_ballot_w64(z != 0.f);
+            // (a lane without a visible key has no sum: m stays -inf)
+            if (!redo && __builtin_amdgcn_ballot_w64(least < kSmallSum && m != -INFINITY)) {
+                uint32_t tiny = 0xFFFFFFFFu;
+                for (int i = 0; i < n_mine; ++i) {
+                    const __amdgpu_buffer_rsrc_t rs = tile_rsrc(vbase, (kt_lo + kKS * i + grp) * kKT);
+                    const uint32_t off = unhoisted(hh) * row_bytes + 16u * col;
+#pragma unroll
+                    for (int j = 0; j < kKT / 2; ++j) {
+                        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 2 * j * row_bytes, 0, 0);
+                        tiny = min(min(tiny, magnitude(v.x)), min(magnitude(v.y), min(magnitude(v.z), magnitude(v.w))));
+                    }
+                }
+                redo = __builtin_amdgcn_ballot_w64(tiny < kTinyMagnitude);
+            }
+            if (redo) {
                 clear();
                 for (int i = 0; i < n_mine; ++i) {
                     floatx16 s;

@@ -115,3 +115,69 @@ def test_prefill_small_chunk_plans(orc, gpu, H, HKV, B, pos0):
                dev[2].data_ptr(), pos.data_ptr(), B, H, HKV, D, gpu.default_scale(), n, None, 0)
     torch.cuda.synchronize()
     _close(out.cpu().numpy(), exact)
+
+
+def _layer(orc, gpu, kernel, H, HKV, B, pos0, seed, qs=1.0, ks=1.0, vs=1.0, edit=None):
+    """One chunk through one of the three prefill kernels: "plain" (rows normed beforehand), "step"
+    (q normed in the attention kernel) or "paged" (32-row blocks in reversed order).  qs and ks scale
+    the norms' gammas (and the past keys), vs all values; edit(k, v, qkv) changes the past rows and the
+    raw chunk.  Returns the output and the operands q, k, v it was computed from."""
+    import torch
+    n, kd = pos0 + B, HKV * D
+    qkv = orc.normal((B, (H + 2 * HKV) * D), seed)
+    k, v = orc.normal((n, HKV, D), seed + 1) * np.float32(ks), orc.normal((n, HKV, D), seed + 2) * np.float32(vs)
+    qkv[:, (H + HKV) * D:] *= np.float32(vs)
+    qg, kg = orc.gamma(D, seed + 3) * np.float32(qs), orc.gamma(D, seed + 4) * np.float32(ks)
+    if edit:
+        edit(k, v, qkv)
+    normed = orc.headnorm_rope(qkv, H, D, qg, pos0, 128, 1e6, 1e-6)
+    normed = orc.headnorm_rope(normed, HKV, D, kg, pos0, 128, 1e6, 1e-6, col0=H * D)
+    q = np.ascontiguousarray(normed[:, :H * D])
+    k[pos0:] = normed[:, H * D:(H + HKV) * D].reshape(B, HKV, D)
+    v[pos0:] = normed[:, (H + HKV) * D:].reshape(B, HKV, D)
+    shape = gpu.AttnShape(H, HKV)
+    ws = gpu.PrefillWorkspace(B, H, HKV, n)
+    if kernel == "plain":
+        return _run(gpu, q, k, v, pos0, H, HKV, ws), q, k, v
+    past_k, past_v = k.copy(), v.copy()
+    past_k[pos0:], past_v[pos0:] = 0, 0
+    kw = {}
+    if kernel == "paged":
+        nblk = (n + 31) // 32
+        table = np.arange(nblk - 1, -1, -1, dtype=np.int32)
+        rows = table[np.arange(n) // 32] * 32 + np.arange(n) % 32
+        pool = np.zeros((2, nblk * 32, HKV, D), np.float32)
+        pool[0, rows], pool[1, rows] = past_k, past_v
+        past_k, past_v = pool
+        kw = dict(block_table=torch.from_numpy(table).cuda(), block_size=32)
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (qkv, past_k, past_v, qg, kg)]
+    pos = torch.tensor([pos0], dtype=torch.int32, device="cuda")
+    out = gpu.prefill_step(dev[0], dev[1].view(-1, kd), dev[2].view(-1, kd), shape, dev[3], dev[4], gpu.rope_table(n),
+                           pos, ws, **kw)
+    torch.cuda.synchronize()
+    return out.cpu().numpy(), q, k, v
+
+
+KERNELS = ["plain", "step", "paged"]
+
+
+@pytest.mark.parametrize("kernel", KERNELS)
+@pytest.mark.parametrize("e", [-112, -118, -124])
+def test_prefill_tiny_values(orc, gpu, kernel, e):
+    """V too small for three bf16 planes (whose smallest step is 2^-133), everywhere and in one column of
+    ordinary values, and a column of zeros.  Same bound as above, column by column: the smallest outputs are
+    fp32 denormals, whose step of 2^-149 is 2^-22 of them."""
+    H, HKV, B, pos0 = 4, 1, 40, 50
+    got, q, k, v = _layer(orc, gpu, kernel, H, HKV, B, pos0, 35000 - e, vs=2.0 ** e)
+    _close(got.astype(np.float64) * 2.0 ** -e, _exact(q, k, v, pos0, H, HKV) * 2.0 ** -e)
+
+    def columns(_, pv, qkv):
+        chunk = qkv[:, (H + HKV) * D:]
+        pv[..., 7] *= np.float32(2.0 ** e)
+        chunk[:, 7] *= np.float32(2.0 ** e)
+        pv[..., 77], chunk[:, 77] = 0, 0
+    got, q, k, v = _layer(orc, gpu, kernel, H, HKV, B, pos0, 35100 - e, edit=columns)
+    exact = _exact(q, k, v, pos0, H, HKV)
+    _close(np.delete(got, 7, axis=-1), np.delete(exact, 7, axis=-1))
+    assert (got[..., 77] == 0).all()
+    _close(got[..., 7].astype(np.float64) * 2.0 ** -e, exact[..., 7] * 2.0 ** -e)
