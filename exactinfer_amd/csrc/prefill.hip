@@ -219,6 +219,10 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t& h, uint32
     l = pk_bf16(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xFFFF0000u));
 }
 constexpr float kPlaneMin = 0x1p-100f;
+// The planes of a small value are off by up to 2^-134, which counts for something only against a large
+// partner.  From this value on an operand is taken to be one, so below it the smallest partner does
+// not matter.
+constexpr float kPlaneMax = 0x1p24f;
 constexpr float kSmallSum = 0x1p-60f;
 // |x| of a nonzero x in an order of its own, zero last: both tests of a value in one comparison
 __device__ __forceinline__ uint32_t magnitude(uint32_t x) { return (x << 1) - 1u; }
@@ -344,6 +348,11 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
         }
     };
     Planes qp[8];
+    // A score on planes is off by at most 2^-134 (|q| + |k|) per element, times the softmax scale: 2^-47
+    // with K below kPlaneMax, q below 2^50 and the scale below 2^30, a larger scale taken off q's limit.
+    // A wave with a q element past it takes its tiles in fp32 after the key loop.
+    const float q_most = __builtin_fabsf(sl2) < 0x1p30f ? 0x1p50f / fmaxf(1.f, __builtin_fabsf(sl2)) : 0.f;
+    uint64_t q_fp32 = 0;
     // raw q rows (kNormQ): QK-norm + RoPE in place, each wave on the 16 rows it staged, 8 lanes
     // per row, two rounds of 8 rows; gamma and both rounds' RoPE rows are loaded (load_norm)
     // while the q rows are still in flight, and used once they have landed (read_q)
@@ -380,10 +389,18 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
         }
         lds_barrier();
         const float* qs = qst + (hw * kQB + col) * kKS_F + 8 * hh;
+        float most = 0.f;
+        if constexpr (kNormQ) {  // a normed and rotated element is at most sqrt(2 * 128) gammas
+#pragma unroll
+            for (int i = 0; i < 16; ++i) most = fmaxf(most, 16.f * __builtin_fabsf(qg[i]));
+        }
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             const float4 x = *reinterpret_cast<const float4*>(qs + 16 * t);
             const float4 y = *reinterpret_cast<const float4*>(qs + 16 * t + 4);
+#pragma unroll
+            for (const float f : {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w})
+                if constexpr (!kNormQ) most = fmaxf(most, __builtin_fabsf(f));
             uint32_t h[4], m[4], l[4];
             split_pair(x.x, x.y, h[0], m[0], l[0]);
             split_pair(x.z, x.w, h[1], m[1], l[1]);
@@ -391,6 +408,7 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
             split_pair(y.z, y.w, h[3], m[3], l[3]);
             qp[t] = {u32x4{h[0], h[1], h[2], h[3]}, u32x4{m[0], m[1], m[2], m[3]}, u32x4{l[0], l[1], l[2], l[3]}};
         }
+        q_fp32 = __builtin_amdgcn_ballot_w64(!(most < q_most));
     };
     const int u_second = nu - 1 - pair;  // the pass-1 unit (none when it equals pair)
     // this workgroup's share of the pair (prefill_share); wave-uniform: readfirstlane keeps the
@@ -455,9 +473,18 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
                 rg[2 * j] = __uint_as_float(v.x), rg[2 * j + 1] = __uint_as_float(v.y);
             }
         };
+        // a value of rg past kPlaneMax turns one of them into NaN, which reaches a sum of every wave that
+        // multiplies it (ten operations; a branch would spill)
+        auto check_planes = [&]() {
+            float most = 0.f;
+#pragma unroll
+            for (int j = 0; j < 16; ++j) most = fmaxf(most, __builtin_fabsf(rg[j]));
+            rg[0] = most < kPlaneMax ? rg[0] : __builtin_nanf("");
+        };
         // half x of the conversion of rg: eight values, one 16-byte piece of each plane
         auto conv_k = [&](int x) {
             uint32_t ch[4], cm[4], cl[4];
+            if (x == 0) check_planes();
 #pragma unroll
             for (int j = 0; j < 4; ++j) split_pair(rg[8 * x + 2 * j], rg[8 * x + 2 * j + 1], ch[j], cm[j], cl[j]);
             char* p = kpl + (8 * hw + (lane >> 3)) * kKRowB + 16 * (lane & 7) + 128 * x;
@@ -532,22 +559,66 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
                 lsum += s[r];
             }
         };
-        // The same two products in fp32 from the cache (q = h + m + l is exact), for a wave whose
-        // planes gave something not finite: see after the key loop.
+        // The same two products in fp32 from the cache, for a wave that planes do not serve: see after the
+        // key loop.  q comes from its row again, normed as in norm_rope_q8 if it is raw (each lane holds the
+        // pairs (d, d + 64) of half its query's elements); values 16t + 8hh .. + 7 take the registers of
+        // planes h and m.
+        auto q_whole = [&]() {
+            const int ln = unhoisted(lane), e0 = 8 * (ln >> 5);
+            const int bq = min(qb * kQB + (ln & 31), B - 1);
+            const float* row = q + (size_t)bq * q_stride + (size_t)h * D + e0;
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                qp[t].h = *reinterpret_cast<const u32x4*>(row + 16 * t);
+                qp[t].m = *reinterpret_cast<const u32x4*>(row + 16 * t + 4);
+            }
+            if constexpr (kNormQ) {
+#pragma clang fp contract(off)
+                double ss = 0.0;
+#pragma unroll
+                for (int t = 0; t < 8; ++t)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const double x = __uint_as_float(qp[t].h[j]), y = __uint_as_float(qp[t].m[j]);
+                        ss = __builtin_fma(x, x, ss);
+                        ss = __builtin_fma(y, y, ss);
+                    }
+                ss += lane_xor_f64<32>(ss);
+                const float inv = (float)(1.0 / sqrt(ss / (double)kHeadDim + (double)eps));
+                const float2* tr = cs + (size_t)(pos0 + bq) * (kHeadDim / 2) + e0;
+                auto turn = [&](uint32_t& lo, uint32_t& hi, int d) {  // elements d + 8hh and 64 further on
+                    const float2 t = tr[d];
+                    const float a = (__uint_as_float(lo) * inv) * q_gamma[d + e0];
+                    const float e = (__uint_as_float(hi) * inv) * q_gamma[64 + d + e0];
+                    const float ac = a * t.x, es = e * t.y, as = a * t.y, ec = e * t.x;
+                    lo = __float_as_uint(ac - es), hi = __float_as_uint(as + ec);
+                };
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        uint32_t lo = qp[t].h[j], hi = qp[t + 4].h[j];
+                        turn(lo, hi, 16 * t + j);
+                        qp[t].h[j] = lo, qp[t + 4].h[j] = hi;
+                        lo = qp[t].m[j], hi = qp[t + 4].m[j];
+                        turn(lo, hi, 16 * t + 4 + j);
+                        qp[t].m[j] = lo, qp[t + 4].m[j] = hi;
+                    }
+            }
+        };
         auto qk_fp32 = [&](int i, floatx16& s) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) s[r] = 0.f;
             const __amdgpu_buffer_rsrc_t rs = tile_rsrc(kbase, (kt_lo + kKS * i + grp) * kKT);
-            const uint32_t off = unhoisted(col) * row_bytes + 32u * hh;
+            const int ln = unhoisted(lane);
+            const uint32_t off = (ln & 31) * row_bytes + 32u * (ln >> 5);
 #pragma unroll
             for (int t = 0; t < 8; ++t) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {  // d = 16t + 8hh + 2j and the next
                     const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rs, off + 64 * t + 8 * j, 0, 0);
-                    const uint32_t h = unhoisted(qp[t].h[j]), m = unhoisted(qp[t].m[j]), l = unhoisted(qp[t].l[j]);
-                    const float q0 = (__uint_as_float(h << 16) + __uint_as_float(m << 16)) + __uint_as_float(l << 16);
-                    const float q1 = (__uint_as_float(h & 0xFFFF0000u) + __uint_as_float(m & 0xFFFF0000u)) +
-                                     __uint_as_float(l & 0xFFFF0000u);
+                    const u32x4 qv = j < 2 ? qp[t].h : qp[t].m;
+                    const float q0 = __uint_as_float(qv[2 * (j & 1)]), q1 = __uint_as_float(qv[2 * (j & 1) + 1]);
                     s = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(v.x), q0, s, 0, 0, 0);
                     s = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(v.y), q1, s, 0, 0, 0);
                 }
@@ -619,12 +690,13 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
 
         // An infinite K or V value (or a finite one past bf16's range) has no planes to multiply:
         // the residual of inf is NaN, and inf times a zero residual is NaN where the fp32 product is
-        // infinite or the key's weight is zero.  Such a tile shows as a sum that is not finite.  A V
-        // value below kPlaneMin may have lost bits of its third plane, which shows only in a sum that is
-        // itself small: weights are at most 2^kLazy and a value is off by at most 2^-134, so over 2^20 keys
-        // a sum from kSmallSum up is off by less than 2^-46 of itself.  A small one has the wave look
-        // through its V tiles, because a column of zeros or of few ordinary values gives one too.  In
-        // both cases the wave then takes its tiles again in fp32, whose outcome stands whatever it is.
+        // infinite or the key's weight is zero.  Such a tile, and one with a K value past kPlaneMax, shows
+        // as a sum that is not finite.  A V value below kPlaneMin may have lost bits of its third plane,
+        // which shows only in a sum that is itself small: weights are at most 2^kLazy and a value is off by
+        // at most 2^-134, so over 2^20 keys a sum from kSmallSum up is off by less than 2^-46 of itself.  A
+        // small one has the wave look through its V tiles, because a column of zeros or of few ordinary
+        // values gives one too.  In both cases, and for a q past its limit, the wave then takes its tiles
+        // again in fp32, whose outcome stands whatever it is.
         {
             float z = lsum * 0.f, least = INFINITY;
 #pragma unroll
@@ -634,7 +706,7 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
                     z = __builtin_fmaf(o[db][r], 0.f, z);
                     least = fminf(least, __builtin_fabsf(o[db][r]));
                 }
-            uint64_t redo = __builtin_amdgcn_ballot_w64(z != 0.f);
+            uint64_t redo = q_fp32 | __builtin_amdgcn_ballot_w64(z != 0.f);
             // (a lane without a visible key has no sum: m stays -inf)
             if (!redo && __builtin_amdgcn_ballot_w64(least < kSmallSum && m != -INFINITY)) {
                 uint32_t tiny = 0xFFFFFFFFu;
@@ -649,8 +721,9 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
                 }
                 redo = __builtin_amdgcn_ballot_w64(tiny < kTinyMagnitude);
             }
-            if (redo) {
+            if (redo && live) {  // (a slot past the last block writes nothing)
                 clear();
+                q_whole();
                 for (int i = 0; i < n_mine; ++i) {
                     floatx16 s;
                     qk_fp32(i, s);

@@ -181,3 +181,24 @@ def test_prefill_tiny_values(orc, gpu, kernel, e):
     _close(np.delete(got, 7, axis=-1), np.delete(exact, 7, axis=-1))
     assert (got[..., 77] == 0).all()
     _close(got[..., 7].astype(np.float64) * 2.0 ** -e, exact[..., 7] * 2.0 ** -e)
+
+
+@pytest.mark.parametrize("kernel", KERNELS)
+@pytest.mark.parametrize("e", [-120, 100, 120])
+def test_prefill_q_out_of_plane_range(orc, gpu, kernel, e):
+    """Tiny q against large K, and K too small for its planes against a q large enough to show it: ordinary
+    scores, same bound."""
+    H, HKV, B, pos0 = 8, 2, 40, 50
+    got, q, k, v = _layer(orc, gpu, kernel, H, HKV, B, pos0, 36000 + e, qs=2.0 ** e, ks=2.0 ** -e)
+    _close(got, _exact(q, k, v, pos0, H, HKV))
+
+
+@pytest.mark.parametrize("split", [False, True])
+def test_prefill_q_past_bf16_range(orc, gpu, split):
+    """A finite q element above bf16's largest value, whose products with small K elements are ordinary."""
+    H, HKV, B, pos0 = 4, 1, 40, 50
+    q, k, v = _inputs(orc, B, pos0, H, HKV, 36500)
+    q[:, 5::D] = np.float32(3.4e38)
+    k[..., 5] *= np.float32(3e-39)
+    got = _run(gpu, q, k, v, pos0, H, HKV, gpu.PrefillWorkspace(B, H, HKV, pos0 + B) if split else None)
+    _close(got, _exact(q, k, v, pos0, H, HKV))
