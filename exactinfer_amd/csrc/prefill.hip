@@ -224,8 +224,11 @@ constexpr float kPlaneMin = 0x1p-100f;
 // not matter.
 constexpr float kPlaneMax = 0x1p24f;
 constexpr float kSmallSum = 0x1p-60f;
-// |x| of a nonzero x in an order of its own, zero last: both tests of a value in one comparison
+// |x| in the order of nonzero values, zero last
 __device__ __forceinline__ uint32_t magnitude(uint32_t x) { return (x << 1) - 1u; }
+__device__ __forceinline__ float of_magnitude(uint32_t m) {  // its |x|; infinite for zero
+    return m == 0xFFFFFFFFu ? INFINITY : __uint_as_float((m >> 1) + 1u);
+}
 constexpr uint32_t kTinyMagnitude = (__builtin_bit_cast(uint32_t, kPlaneMin) << 1) - 1u;
 struct Planes {  // eight values: one MFMA operand per plane
     u32x4 h, m, l;
@@ -494,6 +497,7 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
         };
         auto conv_v = [&](int x) {  // d + x
             uint32_t ch[4], cm[4], cl[4];
+            if (x == 0) check_planes();
 #pragma unroll
             for (int j = 0; j < 4; ++j) split_pair(rg[4 * j + x], rg[4 * j + 2 + x], ch[j], cm[j], cl[j]);
             char* p = vpl + (32 * hw + 2 * (lane & 15) + x) * kVRowB + 16 * (lane >> 4);
@@ -690,13 +694,14 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
 
         // An infinite K or V value (or a finite one past bf16's range) has no planes to multiply:
         // the residual of inf is NaN, and inf times a zero residual is NaN where the fp32 product is
-        // infinite or the key's weight is zero.  Such a tile, and one with a K value past kPlaneMax, shows
-        // as a sum that is not finite.  A V value below kPlaneMin may have lost bits of its third plane,
-        // which shows only in a sum that is itself small: weights are at most 2^kLazy and a value is off by
-        // at most 2^-134, so over 2^20 keys a sum from kSmallSum up is off by less than 2^-46 of itself.  A
-        // small one has the wave look through its V tiles, because a column of zeros or of few ordinary
-        // values gives one too.  In both cases, and for a q past its limit, the wave then takes its tiles
-        // again in fp32, whose outcome stands whatever it is.
+        // infinite or the key's weight is zero.  Such a tile, and one with a K or V value past kPlaneMax,
+        // shows as a sum that is not finite.  A V value or a weight below kPlaneMin may have lost bits of
+        // its third plane, 2^-134: with V below kPlaneMax, weights at most 2^kLazy and 2^20 keys, a sum from
+        // kSmallSum up is off by less than 2^-30 of itself.  A smaller one has the wave look through its V
+        // tiles, because a column of zeros or small V throughout give one too: it stands if no V value is
+        // below kPlaneMin and the largest one is too small for the weights' 2^-134 to show in it.  Otherwise,
+        // and for a q past its limit, the wave takes its tiles again in fp32, whose outcome stands
+        // whatever it is.
         {
             float z = lsum * 0.f, least = INFINITY;
 #pragma unroll
@@ -709,17 +714,31 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
             uint64_t redo = q_fp32 | __builtin_amdgcn_ballot_w64(z != 0.f);
             // (a lane without a visible key has no sum: m stays -inf)
             if (!redo && __builtin_amdgcn_ballot_w64(least < kSmallSum && m != -INFINITY)) {
-                uint32_t tiny = 0xFFFFFFFFu;
+                uint32_t small = 0xFFFFFFFFu, tiny = 0xFFFFFFFFu;  // the smallest nonzero sum and V value
+                if (m != -INFINITY) {
+#pragma unroll
+                    for (int db = 0; db < 4; ++db)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) small = min(small, magnitude(__float_as_uint(o[db][r])));
+                }
+                float most = 0.f;
                 for (int i = 0; i < n_mine; ++i) {
                     const __amdgpu_buffer_rsrc_t rs = tile_rsrc(vbase, (kt_lo + kKS * i + grp) * kKT);
-                    const uint32_t off = unhoisted(hh) * row_bytes + 16u * col;
+                    const int ln = unhoisted(lane);
+                    const uint32_t off = (ln >> 5) * row_bytes + 16u * (ln & 31);
 #pragma unroll
                     for (int j = 0; j < kKT / 2; ++j) {
                         const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 2 * j * row_bytes, 0, 0);
-                        tiny = min(min(tiny, magnitude(v.x)), min(magnitude(v.y), min(magnitude(v.z), magnitude(v.w))));
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            tiny = min(tiny, magnitude(v[e]));
+                            most = fmaxf(most, __builtin_fabsf(__uint_as_float(v[e])));
+                        }
                     }
                 }
-                redo = __builtin_amdgcn_ballot_w64(tiny < kTinyMagnitude);
+                // the sums are off by up to 2^20 2^-134 most; a lane without a nonzero one has nothing to lose
+                const float limit = wave_max(most) * 0x1p-84f;
+                redo = __builtin_amdgcn_ballot_w64(tiny < kTinyMagnitude || limit > of_magnitude(small));
             }
             if (redo && live) {  // (a slot past the last block writes nothing)
                 clear();

@@ -202,3 +202,24 @@ def test_prefill_q_past_bf16_range(orc, gpu, split):
     k[..., 5] *= np.float32(3e-39)
     got = _run(gpu, q, k, v, pos0, H, HKV, gpu.PrefillWorkspace(B, H, HKV, pos0 + B) if split else None)
     _close(got, _exact(q, k, v, pos0, H, HKV))
+
+
+@pytest.mark.parametrize("split", [False, True])
+def test_prefill_tiny_weights_of_huge_values(orc, gpu, split):
+    """Keys of weight near 2^-122 that alone hold a column, with values that make it O(1): the probability
+    keeps its 24 bits.  The scores are exact (one q element), so a weight is off by the exponent's argument:
+    three roundings of about 122 (2^-18 each) times ln 2, 8e-6, and the exponential's own 1e-7."""
+    H, HKV, B, pos0 = 4, 1, 40, 50
+    q, k, v = _inputs(orc, B, pos0, H, HKV, 37000)
+    q[:], k[:] = 0, 0
+    q[:, ::D] = 8
+    cols = list(range(3, 19, 2))
+    v[..., cols] = 0
+    for i, c in enumerate(cols):  # 8 * (120 .. 120.7) * log2(e) / sqrt(128) = 122.4 .. 123.1
+        k[3 * i, 0, 0] = np.float32(-(120.0 + 0.1 * i))
+        v[3 * i, 0, c] = np.float32(2.0 ** 124 * (1 + 0.1 * i))
+    got = _run(gpu, q, k, v, pos0, H, HKV, gpu.PrefillWorkspace(B, H, HKV, pos0 + B) if split else None)
+    exact = _exact(q, k, v, pos0, H, HKV)
+    rest = np.delete(np.arange(D), cols)
+    _close(got[..., rest], exact[..., rest])
+    assert np.max(np.abs(got[..., cols] / exact[..., cols] - 1.0)) <= 1e-5
