@@ -813,7 +813,7 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
 
 // Merge of the ksplit shares of every (query, head): grid ceil(B*H/4), 128 threads; thread
 // = float4 column d4 of row (b, h).  o = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s, empty
-// shares (m = -inf) skipped.
+// shares (m = -inf, l = 0) skipped.
 __global__ __launch_bounds__(128) void k_prefill_combine(const float* __restrict__ part_o,
                                                          const float* __restrict__ part_ml, float* __restrict__ out,
                                                          int rows, int ksplit, const int* __restrict__ pos_dev, int B,
@@ -849,7 +849,8 @@ __global__ __launch_bounds__(128) void k_prefill_combine(const float* __restrict
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int s = 0; s < kPrefillMaxSplit; ++s) {
-        if (s >= ksplit || ml[s].x == -INFINITY) continue;  // an empty share adds nothing
+        // an empty share adds nothing; one whose every score is NaN has m = -inf too, and its NaN l counts
+        if (s >= ksplit || (ml[s].x == -INFINITY && ml[s].y == 0.f)) continue;
         const float wv = __builtin_amdgcn_exp2f(ml[s].x - M);
         L = fmaf(wv, ml[s].y, L);
         o.x = fmaf(wv, v[s].x, o.x);

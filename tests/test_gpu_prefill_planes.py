@@ -223,3 +223,18 @@ def test_prefill_tiny_weights_of_huge_values(orc, gpu, split):
     rest = np.delete(np.arange(D), cols)
     _close(got[..., rest], exact[..., rest])
     assert np.max(np.abs(got[..., cols] / exact[..., cols] - 1.0)) <= 1e-5
+
+
+@pytest.mark.parametrize("B", [2, 33])
+def test_prefill_nan_key_alone_in_its_share(orc, gpu, B):
+    """A NaN key that is the only visible one of its share (one-tile shares, the first query at a tile's
+    first key) makes the row NaN as it does unsplit; rows that do not see it stay finite."""
+    H, HKV, pos0 = 4, 1, 224
+    q, k, v = _inputs(orc, B, pos0, H, HKV, 39000)
+    for t in (pos0, pos0 + 1):
+        kn = k.copy()
+        kn[t, 0, 3] = np.nan
+        plain = _run(gpu, q, kn, v, pos0, H, HKV)
+        split = _run(gpu, q, kn, v, pos0, H, HKV, gpu.PrefillWorkspace(B, H, HKV, pos0 + B))
+        want = np.broadcast_to((np.arange(B) >= t - pos0)[:, None, None], plain.shape)
+        assert (np.isnan(plain) == want).all() and (np.isnan(split) == want).all()
