@@ -603,7 +603,11 @@ static hipError_t launch_t(hipStream_t st, const float* x, long x_stride, const 
         constexpr int kRegs = sizeof(Weights<T, E>) / 4;
         constexpr int kBudget = S::kThreads <= 512 ? 160 : 112;
         constexpr int kFit = (kBudget - S::kVals * NB) / (kRegs + NB);
-        constexpr int kMost = kFit >= 8 ? 8 : kFit >= 6 ? 6 : kFit >= 4 ? 4 : kFit >= 3 ? 3 : 2;
+        // (two activation rows of block formats at ten waves: at most 3.  Graph-timed at 6 or 8 / 3, 6144 outputs
+        // at E 2560 and 7168 at 5120: Q8_0 9.23 / 7.98 and 16.35 / 13.53 us, Q4_K 7.24 / 7.07 and 15.23 / 11.68;
+        // Q6_K at 4 / 3 8.44 / 8.43 and 15.00 / 14.67)
+        constexpr int kTop = T > 1 && NB == 2 && S::kThreads > 512 && kFit > 3 ? 3 : kFit;
+        constexpr int kMost = kTop >= 8 ? 8 : kTop >= 6 ? 6 : kTop >= 4 ? 4 : kTop >= 3 ? 3 : 2;
         const int batches = (turns + kMost - 1) / kMost, want = (turns + batches - 1) / batches;
         constexpr size_t lds = (size_t)NB * S::kHRow * sizeof(float);
         auto go = [&](auto rb) {
