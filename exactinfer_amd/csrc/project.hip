@@ -384,14 +384,16 @@ __global__ __launch_bounds__((RowShape<T, E>::kThreads)) void k_qkv_project(cons
 // With a single activation row the sums need no sharing, and at the hidden sizes whose rows take ten waves
 // above (160 or 320 lanes: 2560 and 5120) a wave per two output rows with every byte of them in flight is
 // the faster layout: four waves to a workgroup, the normed activations read from LDS, no reduction beyond the
-// wave (as it is for F32 at 2048, whose 16 rows a CU are too few to keep rows in flight behind others).  Graph-timed, this against the kernel above: F32 11.35 / 11.63 us at E 2560 and 24.7 / 25.6 at 5120, F16
-// 7.31 / 7.23 and 14.5 / 15.3, Q8_0 7.03 / 7.89 and 14.1 / 14.7, Q4_K 5.86 / 6.40 and 11.0 / 11.4 (Q6_K 8.36 /
-// 8.09 and 18.7 / 15.8: taken above), F32 7.34 / 7.82 at E 2048.
+// wave.  So it is for F32 at 2048, whose 16 rows a CU are too few to keep rows in flight behind others, and
+// for Q4_K at 4096.  Graph-timed on one box, this against the kernel above: F32 11.07 / 11.49 us at E 2560 and
+// 24.36 / 25.50 at 5120, F16 6.72 / 6.98 and 14.47 / 15.00, Q8_0 6.51 / 7.88 and 13.23 / 14.98, Q4_K 5.52 /
+// 6.16 and 11.28 / 11.47; F32 6.79 / 7.43 at 2048; Q4_K 7.82 / 8.22 at 4096, where Q8_0 takes 9.17 / 9.02.
+// Q6_K stays above: staged through LDS like Q8_0 it took 8.09 / 8.13 at 2560 and 18.1 / 15.5 at 5120.
 constexpr int kOneWaves = 4, kOneRows = 2;  // waves per workgroup, rows per wave
 
 template <int T, int E>
 constexpr bool project_one_row() {
-    return (T != 14 && (E == 2560 || E == 5120)) || (T == 0 && E == 2048);
+    return (T != 14 && (E == 2560 || E == 5120)) || (T == 0 && E == 2048) || (T == 12 && E == 4096);
 }
 
 // RMSNorm of the activation row into hs (src/ops.cpp:155-160), kEl elements per thread; the caller's barrier

@@ -13,8 +13,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("wtype", [W_F32, W_F16] + QTYPES)
 @pytest.mark.parametrize("E,n_out,rows", [(1024, 1, 1), (1024, 257, 2), (1024, 2303, 4), (2048, 70, 3), (2048, 4095, 1),
-                                         (2560, 9, 1), (2560, 700, 3), (2560, 1535, 2), (4096, 300, 2), (4096, 1793, 4),
-                                         (5120, 13, 4), (5120, 1025, 1), (5120, 515, 2)])
+                                         (2560, 9, 1), (2560, 700, 3), (2560, 1535, 2), (4096, 300, 2), (4096, 1025, 1),
+                                         (4096, 1793, 4), (5120, 13, 4), (5120, 1025, 1), (5120, 515, 2)])
 def test_projection_partly_filled_launches(orc, gpu, wtype, E, n_out, rows):
     x = orc.normal((rows, E), 8900 + E) * np.float32(3.0)
     gamma = orc.gamma(E, 8901)
