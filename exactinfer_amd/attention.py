@@ -38,12 +38,15 @@ def _need_gpu_f32(name: str, t: torch.Tensor) -> None:
         raise ValueError(f"{name} must be contiguous in its last dimension")
 
 
-@functools.lru_cache(maxsize=None)
+@functools.lru_cache(maxsize=8)
+def _scale_of(head_dim: float) -> float:
+    return float(torch.tensor(1.0, dtype=torch.float32) / torch.sqrt(torch.tensor(head_dim, dtype=torch.float32)))
+
+
 def default_scale(head_dim: int = HEAD_DIM) -> float:
     """1/sqrt(D) rounded to float as the reference does (src/model.cpp:163, src/cuda/model_cuda.cu:1786).
-    A number per head_dim, so it is computed once (4.1 us of tensor operations in every call before)."""
-    return float(torch.tensor(1.0, dtype=torch.float32) / torch.sqrt(torch.tensor(float(head_dim),
-                                                                                  dtype=torch.float32)))
+    Kept by the number: as tensor operations it takes 4.1 us, in every call."""
+    return _scale_of(float(head_dim))
 
 
 @dataclass(frozen=True)

@@ -172,3 +172,17 @@ def test_projection_rows_per_launch():
     L = _capi.lib()
     assert [L.ei_qkv_project_max_rows(e) for e in (1024, 2560, 5120, 6144, 8192, 10240, 24577, 0, -5)] == \
         [4, 4, 4, 4, 3, 2, 0, 0, 0]
+
+
+def test_default_scale_takes_any_number():
+    """default_scale() is kept by the number it is asked for: an array or tensor is one too, and a tensor
+    changed in place is asked for anew."""
+    import torch
+    from exactinfer_amd.attention import default_scale
+    want = float(np.float32(1.0) / np.sqrt(np.float32(128.0)))
+    for d in (128, 128.0, np.array(128), np.float32(128), torch.tensor(128)):
+        assert default_scale(d) == want
+    d = torch.tensor(128.0)
+    assert default_scale(d) == want
+    d.fill_(64.0)
+    assert default_scale(d) == 0.125
