@@ -117,6 +117,10 @@ def test_prefill_small_chunk_plans(orc, gpu, H, HKV, B, pos0):
     _close(out.cpu().numpy(), exact)
 
 
+def _aligned256(n):
+    return (n + 255) & ~255
+
+
 def _layer(orc, gpu, kernel, H, HKV, B, pos0, seed, qs=1.0, ks=1.0, vs=1.0, edit=None):
     """One chunk through one of the three prefill kernels: "plain" (rows normed beforehand), "step"
     (q normed in the attention kernel) or "paged" (32-row blocks in reversed order).  qs and ks scale
@@ -225,6 +229,23 @@ def test_prefill_tiny_weights_of_huge_values(orc, gpu, split):
     assert np.max(np.abs(got[..., cols] / exact[..., cols] - 1.0)) <= 1e-5
 
 
+@pytest.mark.parametrize("kernel", KERNELS)
+def test_prefill_infinities_by_kernel(orc, gpu, kernel):
+    """Infinite, NaN and huge V elements through each kernel: each stays in its own column."""
+    def edit(_, v, __):
+        v[5, 0, 9] = np.float32(3.4e38)
+        v[11, 0, 17] = np.inf
+        v[12, 0, 21] = np.nan
+    for H, HKV in ((4, 1), (5, 1)):
+        got, q, k, v = _layer(orc, gpu, kernel, H, HKV, 70, 60, 38000 + H, edit=edit)
+        with np.errstate(invalid="ignore"):
+            ref = _exact(q, k, v, 60, H, HKV)
+        assert np.isposinf(got[..., 17]).all() and np.isnan(got[..., 21]).all()
+        cols = np.delete(np.arange(D), (9, 17, 21))
+        _close(got[..., cols], ref[..., cols])
+        assert np.max(np.abs(got[..., 9] / ref[..., 9] - 1.0)) <= 1e-5
+
+
 @pytest.mark.parametrize("B", [2, 33])
 def test_prefill_nan_key_alone_in_its_share(orc, gpu, B):
     """A NaN key that is the only visible one of its share (one-tile shares, the first query at a tile's
@@ -238,3 +259,41 @@ def test_prefill_nan_key_alone_in_its_share(orc, gpu, B):
         split = _run(gpu, q, kn, v, pos0, H, HKV, gpu.PrefillWorkspace(B, H, HKV, pos0 + B))
         want = np.broadcast_to((np.arange(B) >= t - pos0)[:, None, None], plain.shape)
         assert (np.isnan(plain) == want).all() and (np.isnan(split) == want).all()
+
+
+def test_prefill_workspace_of_the_coarser_plan(orc, gpu):
+    """A workspace that holds the plan of at least four tiles a share (two shares here) and not the finer
+    one is taken, used within its bytes, and refused when one byte short."""
+    import torch
+    from exactinfer_amd import _capi
+    H, HKV, B, pos0 = 32, 8, 64, 300
+    n, shape = pos0 + B, gpu.AttnShape(32, 8)
+    need = _aligned256(2 * B * H * D * 4) + _aligned256(2 * B * H * 2 * 4)
+    assert need < gpu.PrefillWorkspace(B, H, HKV, n).nbytes
+    buf = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device="cuda")
+    _, q, k, v = _layer(orc, gpu, "plain", H, HKV, B, pos0, 40000)
+    qkv = orc.normal((B, (H + 2 * HKV) * D), 40000)
+    qg, kg = orc.gamma(D, 40003), orc.gamma(D, 40004)
+    exact = _exact(q, k, v, pos0, H, HKV)
+    pos = torch.tensor([pos0], dtype=torch.int32, device="cuda")
+    cs = gpu.rope_table(n)
+
+    def call(step, nbytes):
+        dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (qkv if step else q, k, v, qg, kg)]
+        out = torch.full((B, H, D), float("nan"), dtype=torch.float32, device="cuda")
+        head = (gpu._stream(), dev[0].data_ptr(), dev[0].stride(0), out.data_ptr(), dev[1].data_ptr(),
+                dev[2].data_ptr(), pos.data_ptr(), B, H, HKV, D)
+        tail = (gpu.default_scale(), n, buf.data_ptr(), nbytes)
+        if step:
+            _capi.call("ei_prefill_step", *head, dev[3].data_ptr(), dev[4].data_ptr(), cs.data_ptr(), shape.rope_dim,
+                       float(shape.eps), *tail)
+        else:
+            _capi.call("ei_attn_prefill_split", *head, *tail)
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+
+    for step in (False, True):
+        _close(call(step, need), exact)
+        assert bool((buf[need:] == 0x5A).all())
+        with pytest.raises(Exception, match="workspace"):
+            call(step, need - 1)
