@@ -129,7 +129,8 @@ hipError_t launch_qkv_project(hipStream_t st, const float* x, long x_stride, int
 
 // ------------------------------------------------------------------ prefill.hip
 // Key split across workgroups for short chunks: ksplit shares per query block, merged by a
-// second launch; fixed by (B, max_kv) so graphs replay unchanged.
+// second launch; fixed by B, max_kv and whether the workspace holds the fine plan, so graphs replay
+// unchanged.  (The same call may round differently with a larger workspace.)
 constexpr int kPrefillMaxSplit = 8;
 // fine: shares of as little as one tile (a larger workspace)
 int prefill_split(int B, int H, int HKV, int max_kv, bool fine);

@@ -1,9 +1,11 @@
-// prefill.hip — causal GQA prefill attention on gfx950 bf16 matrix cores, fp32-exact operands.
+// prefill.hip — causal GQA prefill attention on gfx950 bf16 matrix cores, fp32 operands in three planes.
 //
 // Both products run on v_mfma_f32_32x32x16_bf16 (fp32 accumulate; 16x the rate of the fp32
 // 32x32x2 instruction) with every fp32 operand split into three bf16 planes that together hold
-// all of its bits, x = h + m + l.  Six of the nine plane products are taken; the three left out
-// are each at most 2^-27 of |a||b|, an eighth of an fp32 rounding.  An instruction sums 16
+// all of its bits, x = h + m + l (values out of the planes' range are multiplied in fp32: see the
+// split and the check after the key loop).  Six of the nine plane products are taken.  Of the three
+// left out m.l and l.m are at most 2^-25 of |a||b| each and l.l 2^-34: together 2^-24 at worst, an
+// fp32 rounding, and 2^-27.5 in the root mean square over all mantissas.  An instruction sums 16
 // products before it rounds, so a 128-deep score takes 48 roundings, most of them of small
 // terms, against 64 on the fp32 instruction.  Measured error of the output against 64 bits
 // (2-norm): 3.3e-7 against 4.0e-7 with fp32 MFMA (2048-token prompt, H32/HKV8), 4.4e-7 against
@@ -237,10 +239,9 @@ __device__ __forceinline__ floatx16 mfma_bf16(u32x4 a, u32x4 b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
                                                    0, 0);
 }
-// c += a . b to 2^-26 of |a||b|: the six products of planes above that (m.l, l.m and l.l are
-// each at most 2^-27).  a's planes are used up one after another, and next(x) refills plane x
-// (2 l, 1 m, 0 h) with the next step's right after its last use: at least three matrix
-// instructions cover each LDS read, in the registers of one step.
+// c += a . b without m.l, l.m and l.l (together at most 2^-24 of |a||b|).  a's planes are used up one
+// after another, and next(x) refills plane x (2 l, 1 m, 0 h) with the next step's right after its last
+// use: at least three matrix instructions cover each LDS read, in the registers of one step.
 template <typename Next>
 __device__ __forceinline__ void mfma_split(Planes& a, const Planes& b, floatx16& c, Next next) {
     constexpr int kAlu = 0x6;  // VALU and SALU work may move across, LDS reads and MFMAs stay in order
@@ -443,8 +444,7 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
         const int n_mine = (nrange - grp + kKS - 1) / kKS;  // tiles of this key group
 
         // K and V of this group's i-th tile (kt = KS*i + grp): wave hw takes a quarter of each,
-        // 16 floats per lane, into rg, and stores them as planes.  Rows past T repeat the last
-        // visible one (valid memory, masked out).
+        // 16 floats per lane, into rg, and stores them as planes.  Rows past T read as zeros (masked out).
         //   K: row 8*hw + lane/8, d = 8c .. 8c+7 and 64 + 8c .. (c = lane%8): two 16-byte pieces
         //     of a row per plane
         //   V: d = 32*hw + 2*(lane%16) and the next, the eight keys of chunk lane/16 (step s =

@@ -13,18 +13,18 @@
 // contiguous range of output rows.  A row's E weights are spread over the lanes of a row group (L lanes,
 // 8 to 32 weights each; 1 to 8 groups to a workgroup work on different rows), so the normed activations
 // that a lane multiplies by are the same for every row: they are loaded, normed and kept in registers
-// once, and nothing but weights moves after that.  (Read from LDS for every pair of rows, as this kernel
-// did before, they were the bound with several activation rows: each wave read rows x E x 4 bytes for
-// two weight rows, and waited for every read by itself.)  A lane keeps RB rows of weights in flight:
+// once, and nothing but weights moves after that.  (Read from LDS for every pair of rows they bound the
+// kernel with several activation rows: each wave reads rows x E x 4 bytes for two weight rows and waits for
+// every read by itself.)  A lane keeps RB rows of weights in flight:
 // each row's registers are loaded again, with the row RB further on, as soon as they are used, so the
 // stream runs on under the arithmetic.  The partial sums of RB rows x NB activation rows are added over
 // 32 lanes by one transposing butterfly and over the half-waves of the group through LDS.
 //
-// Measured, graph-timed per launch, before -> now (us; a plain read takes 6.2 at 31.5 MB, 11.5 at
-// 67 MB): F16 at E 2560, 6144 outputs, 2 rows 12.6 -> 8.3, 4 rows 24.3 -> 9.9; E 4096, 4 rows 39.4 -> 12.1; E 5120,
-// 7168 outputs, 4 rows 75.3 -> 17.1; F32 there 66.6 -> 26.1; Q8_0 41.3 -> 16.4; Q4_K 40.1 -> 15.5; Q6_K 48.6 ->
-// 17.1; one row of Q6_K at 5120 18.7 -> 15.8; Q4_K at E 1024, 4096 outputs, 4 rows 5.9 -> 4.5.  Several rows cost
-// little more than one now: the stream bounds them, and what is left over it is the launch's start, the norm
+// Measured, graph-timed per launch, activations read from LDS -> this layout (us; a plain read of the weights takes 6.2
+// at 31.5 MB, 8.7 at 50 MB): F16 at E 2560, 6144 outputs, 2 rows 12.3 -> 8.1, 4 rows 24.1 -> 9.6; E 4096, 4 rows 39.0 ->
+// 12.4; E 5120, 7168 outputs, 4 rows 74.8 -> 16.8; F32 there 66.5 -> 25.9; Q8_0 40.7 -> 16.6; Q4_K 40.1 -> 15.4; Q6_K
+// 48.0 -> 17.1; one row of Q6_K at 5120 18.1 -> 15.5; Q4_K at E 1024, 4096 outputs, 4 rows 5.9 -> 4.4.  Several rows cost
+// little more than one: the stream bounds them, and what is left over it is the launch's start, the norm
 // and the last batch's sums.  Tried and not kept: the sums in LDS-read order with four or eight waves a
 // workgroup (F16, E 2560, 4 rows: 14.2), activations loaded lane by lane from memory (16 values a lane, 64
 // bytes apart: Q4_K one row 7.3 against 6.4), two workgroups a CU (8.9), 15 waves (7.8), branches around the
@@ -578,7 +578,7 @@ static int qkv_project_pieces(int E, bool w_f16) {
 bool qkv_project_built(int E, int w_type) {
     if (w_type == 0 || w_type == 1) return qkv_project_pieces(E, w_type == 1) != 0;
     if (w_type != 8 && w_type != 12 && w_type != 14) return false;
-    // the dense Qwen3 hidden sizes (whole 256-value super-blocks, 8-value items per lane)
+    // the dense Qwen3 hidden sizes (whole 256-value super-blocks; a lane's item is 16 values)
     return E == 1024 || E == 2048 || E == 2560 || E == 4096 || E == 5120;
 }
 

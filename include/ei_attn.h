@@ -221,7 +221,10 @@ int ei_decode_step_paged(ei_stream_t stream, const float* qkv, long row_stride, 
  * B query rows (row b at q + b*q_stride, heads [n_head][128], already normed + roped) at
  * positions *pos_dev + b; query b attends to cache rows 0 .. *pos_dev + b (the whole
  * chunk's K/V must already be appended).  out [B][n_head][128].  Matrix-core contraction of
- * fp32 operands (three bf16 planes each, fp32 accumulate) with online softmax.  Replaces k_attn_prefill64 (src/cuda/model_cuda.cu:1204-1341);
+ * fp32 operands (three bf16 planes each, fp32 accumulate) with online softmax.  Operands whose
+ * planes would lose bits are multiplied in fp32, two to three times slower: K or V from 2^24 up,
+ * q times scale from about 2^50 up (with in-kernel q norm: 16 q_gamma), V values below 2^-100 in a
+ * sum that small, infinities and NaN.  Replaces k_attn_prefill64 (src/cuda/model_cuda.cu:1204-1341);
  * the math is the CPU reference's per-token attention (src/model.cpp:138-140, :191-214). */
 int ei_attn_prefill(ei_stream_t stream, const float* q, long q_stride, float* out, const float* kc, const float* vc,
                     const int* pos_dev, int B, int n_head, int n_head_kv, int head_dim, float scale);
@@ -235,7 +238,9 @@ int ei_attn_prefill(ei_stream_t stream, const float* q, long q_stride, float* ou
  * shares with a second launch, using `ws`: ei_attn_prefill_ws_bytes(max_B, ...) bytes serve
  * every chunk of up to max_B rows (0 bytes when no split is planned; the call then equals
  * ei_attn_prefill).  A smaller workspace is taken too if it holds the plan whose shares have at
- * least four 32-key tiles each (none is needed where that plan does not split).  Same semantics and arguments as ei_attn_prefill otherwise; no
+ * least four 32-key tiles each (none is needed where that plan does not split); the two plans add
+ * in another order, so a result's last bits depend on which of them the workspace holds.  Same
+ * semantics and arguments as ei_attn_prefill otherwise; no
  * counterpart in the reference beyond k_attn_prefill64.  Calls sharing `ws` must not overlap. */
 size_t ei_attn_prefill_ws_bytes(int max_B, int n_head, int n_head_kv, int max_kv);
 int ei_attn_prefill_split(ei_stream_t stream, const float* q, long q_stride, float* out, const float* kc,

@@ -400,7 +400,7 @@ def test_prefill_step_matches_reference(orc, gpu, H, HKV, B, pos0, max_kv, rope_
     """ei_prefill_step == headnorm_rope(Q), headnorm_rope(K), append, reference attention:
     cache rows and the in-place K heads bit-exact, attention within ATTN_RTOL; the Q heads stay
     raw in qkv when the kernel norms them itself and are normed in place otherwise (rope_dim 64,
-    or a plan of more than two key shares, takes the prologue for every head)."""
+    or a plan of more than four key shares of at least four tiles, takes the prologue for every head)."""
     shape = gpu.AttnShape(H, HKV, rope_dim=rope_dim)
     n_ctx = max(max_kv, pos0 + B)
     k, v = _cache(orc, n_ctx, HKV, 1500 + B)
@@ -419,7 +419,7 @@ def test_prefill_step_matches_reference(orc, gpu, H, HKV, B, pos0, max_kv, rope_
     got = _host(buf)
     assert bits_equal(got[:, H * D:], normed[:, H * D:])
     # Q heads: raw when the kernel norms them itself, normed in place when the prologue did
-    # (partial rope_dim, or a plan of more than two key shares)
+    # (partial rope_dim, or a plan of more than four key shares of at least four tiles)
     q_raw = bits_equal(got[:, :H * D], qkv[:, :H * D])
     assert q_raw or bits_equal(got[:, :H * D], normed[:, :H * D])
     if rope_dim != D:

@@ -1,5 +1,6 @@
 """GPU tests of the prefill kernel's three-plane products: every fp32 K, V, Q and P value is
-multiplied as three bf16 planes that together hold all its bits.  Sizes sit at the edges of the
+multiplied as three bf16 planes that together hold all its bits, or in fp32 where it is out of the
+planes' range.  Sizes sit at the edges of the
 tiles (32 keys, 32-query blocks, units of 4 slots, two key groups), values at the edges of the
 planes' range."""
 import numpy as np
@@ -61,8 +62,8 @@ def test_prefill_error_against_float64(orc, gpu, H, HKV, B, pos0):
 
 
 def test_prefill_small_and_large_magnitudes(orc, gpu):
-    """Planes keep fp32's exponent range: values near 1e-33 keep all their bits, and K near the
-    largest float against tiny q gives ordinary scores.  Same bound as above."""
+    """V near 1e-33, and K near 1e30 against q near 1e-30, which gives ordinary scores.  Same bound as
+    above."""
     H, HKV, B, pos0 = 4, 1, 40, 50
     q, k, v = _inputs(orc, B, pos0, H, HKV, 32000)
     got = _run(gpu, q * np.float32(2.0 ** -100), k * np.float32(2.0 ** 100), v * np.float32(2.0 ** -110), pos0, H, HKV)
