@@ -49,12 +49,13 @@
 // raised wave priority of the softmax half, whose chain is the longer one, another 3%).  Each
 // matrix step refills its three LDS operands right after their last use (mfma_split).
 //
-// What bounds it: the matrix power of the part.  At 8192 tokens (H32/HKV8) the kernel runs 217
-// TFLOP/s of attention = 1.30 PFLOP/s of bf16 MFMA at 1.65 GHz (the clock gives way under bf16
+// What bounds it: the matrix power of the part.  At 8192 tokens (H32/HKV8) the kernel runs 211
+// TFLOP/s of attention = 1.27 PFLOP/s of bf16 MFMA at 1.65 GHz (the clock gives way under bf16
 // load: a bare register-to-register MFMA loop on random bits reaches 1.53-1.63 PFLOP/s at
-// 1.6-1.66 GHz), against 139 TFLOP/s on fp32 MFMA; 2048 tokens 285 -> 188 us a step, 512 tokens
-// at 7680 (H16/HKV8) 268 -> 160 us.  With parts taken out (timing only): without the K/V split
-// and its loads 2.14 ms of 2.53, without the loads alone 2.38, without operand reads as well as
+// 1.6-1.66 GHz), against 139 TFLOP/s on fp32 MFMA; 2048 tokens 285 -> 193 us a step, 512 tokens
+// at 7680 (H16/HKV8) 268 -> 164 us.  The checks of the planes' range are 1.2 to 1.9% of that (2-3%
+// of a small chunk).  With parts taken out (timing only, before those checks): without the K/V
+// split and its loads 2.14 ms of 2.53, without the loads alone 2.38, without operand reads as well as
 // the split 2.04, without the exponentials too 1.98.
 //
 // q and the output pass through LDS too, so that global memory sees whole 512-byte rows:
