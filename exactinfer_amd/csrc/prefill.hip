@@ -141,6 +141,20 @@ constexpr int kLdsF = kQStageF + kSlots * kQB * kKS_F;
 static_assert(kKS * 3 * kKPlane <= kQStageF * 4, "K planes below the staging area");
 static_assert(kQStageF * 4 + kKS * 3 * kVPlane <= kLdsF * 4, "V planes within the LDS span");
 
+// A value the optimiser may not carry across loop iterations: what is derived from it is computed
+// where it is used (the vector registers of the key loop are full, hoisted addresses would spill).
+__device__ __forceinline__ int unhoisted(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+__device__ __forceinline__ float here(float x) {  // the same of a kernel argument
+    asm volatile("" : "+s"(x));
+    return x;
+}
+__device__ __forceinline__ float uniform(float x) {  // a wave-uniform value, in a scalar register
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
+}
+
 // QK-norm + RoPE of two q rows in LDS (rope_dim = 128), eight lanes per row: lane k of a row
 // holds elements 8k..8k+7 and their rotate-half partners 64+8k..64+8k+7.  Same arithmetic as the
 // prologue's head-norm, which follows the reference CPU path (rmsnorm, src/ops.cpp:155-160; rope,
@@ -174,7 +188,7 @@ __device__ __forceinline__ void norm_rope_q8(float* row0, float* row1, const flo
         ss += lane_xor_f64<1>(ss);
         ss += lane_xor_f64<2>(ss);
         ss += lane_xor_f64<4>(ss);
-        inv[h] = (float)(1.0 / sqrt(ss / (double)kHeadDim + (double)eps));
+        inv[h] = (float)(1.0 / sqrt(ss / (double)kHeadDim + (double)here(eps)));
     }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -263,13 +277,6 @@ __device__ __forceinline__ void mfma_split(Planes& a, const Planes& b, floatx16&
     __builtin_amdgcn_sched_barrier(kAlu);
 }
 
-// A value the optimiser may not carry across loop iterations: what is derived from it is computed
-// where it is used (the vector registers of the key loop are full, hoisted addresses would spill).
-__device__ __forceinline__ int unhoisted(int x) {
-    asm volatile("" : "+v"(x));
-    return x;
-}
-
 // kPaged: key t of the sequence sits in pool row btab[t >> bshift] << bshift | (t & mask), the
 // block size 2^bshift >= 32, so a 32-key tile lies in one block and its rows are consecutive.
 template <bool kNormQ, bool kPaged>
@@ -356,7 +363,7 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
     // A score on planes is off by at most 2^-134 (|q| + |k|) per element, times the softmax scale: 2^-47
     // with K below kPlaneMax, q below 2^50 and the scale below 2^30, a larger scale taken off q's limit.
     // A wave with a q element past it takes its tiles in fp32 after the key loop.
-    const float q_most = __builtin_fabsf(sl2) < 0x1p30f ? 0x1p50f / fmaxf(1.f, __builtin_fabsf(sl2)) : 0.f;
+    const float q_scale = uniform(__builtin_fabsf(sl2) < 0x1p30f ? fmaxf(1.f, __builtin_fabsf(sl2)) : INFINITY);
     uint64_t q_fp32 = 0;
     // raw q rows (kNormQ): QK-norm + RoPE in place, each wave on the 16 rows it staged, 8 lanes
     // per row, two rounds of 8 rows; gamma and both rounds' RoPE rows are loaded (load_norm)
@@ -367,7 +374,7 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
         if constexpr (kNormQ) {
             int r0, jm, hq;
             stage_rows(u, r0, jm, hq);
-            const int k = lane & 7, j = lane >> 3;
+            const int ln = unhoisted(lane), k = ln & 7, j = ln >> 3;
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const float4 ga = *reinterpret_cast<const float4*>(q_gamma + 8 * k + 4 * i);
@@ -413,7 +420,7 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
             split_pair(y.z, y.w, h[3], m[3], l[3]);
             qp[t] = {u32x4{h[0], h[1], h[2], h[3]}, u32x4{m[0], m[1], m[2], m[3]}, u32x4{l[0], l[1], l[2], l[3]}};
         }
-        q_fp32 = __builtin_amdgcn_ballot_w64(!(most < q_most));
+        q_fp32 = __builtin_amdgcn_ballot_w64(!(most * q_scale < 0x1p50f));
     };
     const int u_second = nu - 1 - pair;  // the pass-1 unit (none when it equals pair)
     // this workgroup's share of the pair (prefill_share); wave-uniform: readfirstlane keeps the
@@ -483,7 +490,7 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
             float most = 0.f;
 #pragma unroll
             for (int j = 0; j < 16; ++j) most = fmaxf(most, __builtin_fabsf(rg[j]));
-            rg[0] = most < kPlaneMax ? rg[0] : __builtin_nanf("");
+            rg[0] = most < kPlaneMax ? rg[0] : __uint_as_float(0xFFFFFFFFu);  // (a NaN that is an inline constant)
         };
         // half x of the conversion of rg: eight values, one 16-byte piece of each plane
         auto conv_k = [&](int x) {
@@ -589,7 +596,7 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
                         ss = __builtin_fma(y, y, ss);
                     }
                 ss += lane_xor_f64<32>(ss);
-                const float inv = (float)(1.0 / sqrt(ss / (double)kHeadDim + (double)eps));
+                const float inv = (float)(1.0 / sqrt(ss / (double)kHeadDim + (double)here(eps)));
                 const float2* tr = cs + (size_t)(pos0 + bq) * (kHeadDim / 2) + e0;
                 auto turn = [&](uint32_t& lo, uint32_t& hi, int d) {  // elements d + 8hh and 64 further on
                     const float2 t = tr[d];
@@ -799,14 +806,14 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
             const int sl = kSlots * u + (wu >> 1);  // wave wu stores rows 16*(wu&1).. of slot wu/2
             const int qbo = fdiv(sl, fG), ho = kvh * G + sl - qbo * G;
             float* dst0 = ksplit == 1 ? out : part_o + (size_t)split * B * H * D;
-            const int hh0 = unhoisted(hh);
+            const int ln = unhoisted(lane), hh0 = ln >> 5, c4 = 4 * (ln & 31);
 #pragma unroll
             for (int j = 0; j < kQB / 4; ++j) {
                 const int jj = (kQB / 2) * (wu & 1) + 2 * j + hh0;
                 const int bo = qbo * kQB + jj;
-                const float4 v = *reinterpret_cast<const float4*>(qst + ((wu >> 1) * kQB + jj) * kKS_F + 4 * col);
+                const float4 v = *reinterpret_cast<const float4*>(qst + ((wu >> 1) * kQB + jj) * kKS_F + c4);
                 if (sl < nslot && bo < B)
-                    *reinterpret_cast<float4*>(dst0 + ((size_t)bo * H + ho) * D + 4 * col) = v;
+                    *reinterpret_cast<float4*>(dst0 + ((size_t)bo * H + ho) * D + c4) = v;
             }
         }
     }
