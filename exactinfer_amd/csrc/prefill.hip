@@ -706,22 +706,25 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
         // shows as a sum that is not finite.  A V value or a weight below kPlaneMin may have lost bits of
         // its third plane, 2^-134: with V below kPlaneMax, weights at most 2^kLazy and 2^20 keys, a sum from
         // kSmallSum up is off by less than 2^-30 of itself.  A smaller one has the wave look through its V
-        // tiles, because a column of zeros or small V throughout give one too: it stands if no V value is
-        // below kPlaneMin and the largest one is too small for the weights' 2^-134 to show in it.  Otherwise,
-        // and for a q past its limit, the wave takes its tiles again in fp32, whose outcome stands
-        // whatever it is.
+        // tiles, in the blocks of 32 columns with such a sum, because a column of zeros or small V throughout
+        // give one too (8192 tokens: 10% with one column of zeros): it stands if no V value there is below
+        // kPlaneMin and the largest one is too small for the weights' 2^-134 to show in it.  Otherwise, and
+        // for a q past its limit, the wave takes its tiles again in fp32, whose outcome stands whatever it is.
         {
-            float z = lsum * 0.f, least = INFINITY;
+            float z = lsum * 0.f, least[4];  // per block of 32 columns
 #pragma unroll
-            for (int db = 0; db < 4; ++db)
+            for (int db = 0; db < 4; ++db) {
+                least[db] = INFINITY;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     z = __builtin_fmaf(o[db][r], 0.f, z);
-                    least = fminf(least, __builtin_fabsf(o[db][r]));
+                    least[db] = fminf(least[db], __builtin_fabsf(o[db][r]));
                 }
+            }
+            const float least_all = fminf(fminf(least[0], least[1]), fminf(least[2], least[3]));
             uint64_t redo = q_fp32 | __builtin_amdgcn_ballot_w64(z != 0.f);
             // (a lane without a visible key has no sum: m stays -inf)
-            if (!redo && __builtin_amdgcn_ballot_w64(least < kSmallSum && m != -INFINITY)) {
+            if (!redo && __builtin_amdgcn_ballot_w64(least_all < kSmallSum && m != -INFINITY)) {
                 uint32_t small = 0xFFFFFFFFu, tiny = 0xFFFFFFFFu;  // the smallest nonzero sum and V value
                 if (m != -INFINITY) {
 #pragma unroll
@@ -730,17 +733,21 @@ __global__ __launch_bounds__(64 * kSlots * kKS) void k_prefill(const float* __re
                         for (int r = 0; r < 16; ++r) small = min(small, magnitude(__float_as_uint(o[db][r])));
                 }
                 float most = 0.f;
-                for (int i = 0; i < n_mine; ++i) {
-                    const __amdgpu_buffer_rsrc_t rs = tile_rsrc(vbase, (kt_lo + kKS * i + grp) * kKT);
-                    const int ln = unhoisted(lane);
-                    const uint32_t off = (ln >> 5) * row_bytes + 16u * (ln & 31);
 #pragma unroll
-                    for (int j = 0; j < kKT / 2; ++j) {
-                        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 2 * j * row_bytes, 0, 0);
+                for (int db = 0; db < 4; ++db) {
+                    if (!__builtin_amdgcn_ballot_w64(least[db] < kSmallSum && m != -INFINITY)) continue;
+                    for (int i = 0; i < n_mine; ++i) {
+                        const __amdgpu_buffer_rsrc_t rs = tile_rsrc(vbase, (kt_lo + kKS * i + grp) * kKT);
+                        const int ln = unhoisted(lane);
+                        const uint32_t off = (ln >> 3) * row_bytes + 16u * (ln & 7) + 128u * db;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            tiny = min(tiny, magnitude(v[e]));
-                            most = fmaxf(most, __builtin_fabsf(__uint_as_float(v[e])));
+                        for (int j = 0; j < kKT / 8; ++j) {
+                            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 8 * j * row_bytes, 0, 0);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                tiny = min(tiny, magnitude(v[e]));
+                                most = fmaxf(most, __builtin_fabsf(__uint_as_float(v[e])));
+                            }
                         }
                     }
                 }
