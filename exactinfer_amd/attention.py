@@ -9,7 +9,6 @@ The names follow the reference's per-layer attention steps (src/cuda/model_cuda.
 """
 from __future__ import annotations
 
-import functools
 from dataclasses import dataclass
 
 import torch
@@ -38,15 +37,17 @@ def _need_gpu_f32(name: str, t: torch.Tensor) -> None:
         raise ValueError(f"{name} must be contiguous in its last dimension")
 
 
-@functools.lru_cache(maxsize=8)
 def _scale_of(head_dim: float) -> float:
-    return float(torch.tensor(1.0, dtype=torch.float32) / torch.sqrt(torch.tensor(head_dim, dtype=torch.float32)))
+    one, d = torch.tensor((1.0, head_dim), dtype=torch.float32, device="cpu")
+    return float(one / torch.sqrt(d))
+
+
+_SCALE = _scale_of(float(HEAD_DIM))  # made once: as tensor operations it takes 4 us, in every call
 
 
 def default_scale(head_dim: int = HEAD_DIM) -> float:
-    """1/sqrt(D) rounded to float as the reference does (src/model.cpp:163, src/cuda/model_cuda.cu:1786).
-    Kept by the number: as tensor operations it takes 4.1 us, in every call."""
-    return _scale_of(float(head_dim))
+    """1/sqrt(D) rounded to float as the reference does (src/model.cpp:163, src/cuda/model_cuda.cu:1786)."""
+    return _SCALE if head_dim is HEAD_DIM else _scale_of(float(head_dim))
 
 
 @dataclass(frozen=True)

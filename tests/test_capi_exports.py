@@ -175,8 +175,8 @@ def test_projection_rows_per_launch():
 
 
 def test_default_scale_takes_any_number():
-    """default_scale() is kept by the number it is asked for: an array or tensor is one too, and a tensor
-    changed in place is asked for anew."""
+    """default_scale() keeps no answer by an argument's identity: an array or tensor is a number too, and a
+    tensor changed in place gives the new one."""
     import torch
     from exactinfer_amd.attention import default_scale
     want = float(np.float32(1.0) / np.sqrt(np.float32(128.0)))
