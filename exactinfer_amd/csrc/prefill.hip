@@ -49,12 +49,11 @@
 // raised wave priority of the softmax half, whose chain is the longer one, another 3%).  Each
 // matrix step refills its three LDS operands right after their last use (mfma_split).
 //
-// What bounds it: the matrix power of the part.  At 8192 tokens (H32/HKV8) the kernel runs 211
-// TFLOP/s of attention = 1.27 PFLOP/s of bf16 MFMA at 1.65 GHz (the clock gives way under bf16
+// What bounds it: the matrix power of the part.  At 8192 tokens (H32/HKV8) the kernel runs 219
+// TFLOP/s of attention = 1.31 PFLOP/s of bf16 MFMA at 1.65 GHz (the clock gives way under bf16
 // load: a bare register-to-register MFMA loop on random bits reaches 1.53-1.63 PFLOP/s at
-// 1.6-1.66 GHz), against 139 TFLOP/s on fp32 MFMA; 2048 tokens 285 -> 193 us a step, 512 tokens
-// at 7680 (H16/HKV8) 268 -> 164 us.  The checks of the planes' range are 1.2 to 1.9% of that (2-3%
-// of a small chunk).  With parts taken out (timing only, before those checks): without the K/V
+// 1.6-1.66 GHz), against 139 TFLOP/s on fp32 MFMA; 2048 tokens 285 -> 187 us a step, 512 tokens
+// at 7680 (H16/HKV8) 268 -> 163 us.  The checks of the planes' range are 0-2% of that.  With parts taken out (timing only, before those checks): without the K/V
 // split and its loads 2.14 ms of 2.53, without the loads alone 2.38, without operand reads as well as
 // the split 2.04, without the exponentials too 1.98.
 //
