@@ -385,7 +385,7 @@ __global__ __launch_bounds__((RowShape<T, E>::kThreads)) void k_qkv_project(cons
 // above (160 or 320 lanes: 2560 and 5120) a wave per two output rows with every byte of them in flight is
 // the faster layout: four waves to a workgroup, the normed activations read from LDS, no reduction beyond the
 // wave.  So it is for F32 at 2048, whose 16 rows a CU are too few to keep rows in flight behind others, and
-// for Q4_K at 4096.  Graph-timed on one box, this against the kernel above: F32 11.07 / 11.49 us at E 2560 and
+// for Q4_K at 4096.  Graph-timed in one run, this against the kernel above: F32 11.07 / 11.49 us at E 2560 and
 // 24.36 / 25.50 at 5120, F16 6.72 / 6.98 and 14.47 / 15.00, Q8_0 6.51 / 7.88 and 13.23 / 14.98, Q4_K 5.52 /
 // 6.16 and 11.28 / 11.47; F32 6.79 / 7.43 at 2048; Q4_K 7.82 / 8.22 at 4096, where Q8_0 takes 9.17 / 9.02.
 // Q6_K stays above: staged through LDS like Q8_0 it took 8.09 / 8.13 at 2560 and 18.1 / 15.5 at 5120.
